@@ -3,7 +3,7 @@
 // translation unit per padded size so that the heavily unrolled
 // instantiations compile in parallel.
 #pragma once
-#include "nrocm_internal.hpp"
+#include "exact_div.hpp"
 
 namespace nrocm_chol {
 
@@ -297,40 +297,10 @@ __device__ __forceinline__ void backward(const double *L, int lda, double (&b)[C
 
 // ------------------------------------------------------------ fused factor + solve
 
-// Exact division with a reciprocal reused across numerators.  hipcc expands an
-// f64 x / d as s = div_scale(d), y = rcp(s) refined by two Newton steps,
-// q0 = x' * y, r = fma(-s, q0, x'), q = div_fmas(r, y, q0), div_fixup(q, d, x).
-// When 2^-100 <= |d| <= 2^100 and 2^-900 <= |x| <= 2^600 both scalings are
-// identities, div_fmas is a plain fma and the fixup returns q unchanged, so
-// div_with(x, d, recip_refined(d)) is bit-identical to x / d.  Outside that
-// range (zeros, infinities, NaNs, extreme exponents) callers use x / d.
-__device__ __forceinline__ double recip_refined(double d)
-{
-    const double r0 = __builtin_amdgcn_rcp(d);
-    const double e0 = __builtin_fma(-d, r0, 1.0);
-    const double r1 = __builtin_fma(r0, e0, r0);
-    const double e1 = __builtin_fma(-d, r1, 1.0);
-    return __builtin_fma(r1, e1, r1);
-}
-
-__device__ __forceinline__ double div_with(double x, double d, double y)
-{
-    const double q0 = x * y;
-    const double rem = __builtin_fma(-d, q0, x);
-    return __builtin_fma(rem, y, q0);
-}
-
-__device__ __forceinline__ bool div_den_ok(double d)
-{
-    const double ad = __builtin_fabs(d);
-    return ad >= 0x1p-100 && ad <= 0x1p100;
-}
-
-__device__ __forceinline__ bool div_num_ok(double x)
-{
-    const double ax = __builtin_fabs(x);
-    return ax >= 0x1p-900 && ax <= 0x1p600;
-}
+using nrocm_div::div_den_ok;
+using nrocm_div::div_num_ok;
+using nrocm_div::div_with;
+using nrocm_div::recip_refined;
 
 // a[i] for a wavefront-uniform i (a scalar branch tree, no scratch).
 template <int NB>

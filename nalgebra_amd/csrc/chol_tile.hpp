@@ -34,6 +34,7 @@ namespace nrocm_chol_tile {
 using nrocm_chol::div_den_ok;
 using nrocm_chol::div_with;
 using nrocm_chol::lane_value;
+using nrocm_div::num_in_range;
 using nrocm_chol::recip_refined;
 
 constexpr int MAXRHS = 4;  // right-hand sides carried through the factor (one per lane row)
@@ -93,15 +94,6 @@ __device__ __forceinline__ void upd(double &acc, double x, double y)
     } else {
         asm("v_fma_f64 %0, -%1, %2, %0" : "+v"(acc) : "v"(x), "v"(y));
     }
-}
-
-// Numerator range of div_with from the exponent field alone: 2^-900 <= |x| <
-// 2^600, or +0 (for which the three-instruction form also gives +0).
-__device__ __forceinline__ bool num_in_range(double x)
-{
-    const unsigned long long b = (unsigned long long)__double_as_longlong(x);
-    const unsigned e = (unsigned)(b >> 52) & 0x7ffu;
-    return (e - 123u) <= 1499u || b == 0ull;
 }
 
 // Exact quotient v / den for a wavefront-uniform den with reciprocal y: the

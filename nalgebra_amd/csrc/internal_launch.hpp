@@ -38,13 +38,18 @@ int nrocm_getrf_window_s(nrocm_handle h, int n, float *A, int lda, int *ipiv, in
 int nrocm_potrf_small(nrocm_handle h, int n, double *a, int lda, double *b, int ldb, int nrhs, int *info,
                       bool exact, double substitute = 0.0);
 
-// solve_lookback.hip: LU::solve_mut for any n, one 64-row block per workgroup.
-// Scratch: nrocm_getrs_scratch_bytes(n) bytes of device memory; allocates nothing.
-constexpr int NROCM_GETRS_LOOKBACK_MIN = 1024;  // nrocm_dgetrs uses it from this n on
-size_t nrocm_getrs_scratch_bytes(int n);
-int nrocm_getrs_lookback(nrocm_handle h, hipStream_t st, int n, int nrhs, const double *lu, int lda, const int *ipiv,
-                         double *b, int ldb, int *info, bool exact, void *scratch);
-// Cholesky::solve_mut for large n (nrocm_dpotrs from NROCM_GETRS_LOOKBACK_MIN on),
-// same scratch size.
-int nrocm_potrs_lookback(nrocm_handle h, hipStream_t st, int n, int nrhs, const double *L, int lda, double *b,
-                         int ldb, bool exact, void *scratch);
+// solve_small.hip: LU::solve_mut, Cholesky::solve_mut and QR::solve_mut's
+// upper solve, each in one launch that shares nothing with other calls.
+constexpr int NROCM_GETRS_LOOKBACK_MIN = 1024;  // LU and Cholesky solves of this n on go to solve_lookback.hip
+int nrocm_getrs_small(nrocm_handle h, int n, int nrhs, const double *lu, int lda, const int *ipiv, double *b, int ldb,
+                      int *info, bool exact);
+int nrocm_potrs_small(nrocm_handle h, int n, int nrhs, const double *l, int lda, double *b, int ldb, bool exact);
+int nrocm_qr_rsolve(nrocm_handle h, int n, int nrhs, const double *qr, int lda, const double *diag, double *b, int ldb,
+                    int *info);
+
+// solve_lookback.hip: the same solves for any n on many workgroups, in the handle's workspace.
+int nrocm_getrs_lookback(nrocm_handle h, int n, int nrhs, const double *lu, int lda, const int *ipiv, double *b,
+                         int ldb, int *info, bool exact);
+int nrocm_potrs_lookback(nrocm_handle h, int n, int nrhs, const double *L, int lda, double *b, int ldb, bool exact);
+int nrocm_qr_rsolve_lookback(nrocm_handle h, int n, int nrhs, const double *qr, int lda, const double *diag, double *b,
+                             int ldb, int *info);

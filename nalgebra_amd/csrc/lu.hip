@@ -165,61 +165,6 @@ int getrf_impl(nrocm_handle h, hipStream_t st, int m, int n, T *A, int lda, int 
     return NROCM_OK;
 }
 
-// ---------------------------------------------------------------- getrs (one workgroup)
-// LU::solve_mut (lu.rs:242-260): swaps, unit-lower forward solve
-// (solve.rs:106-133), upper backward solve (solve.rs:137-182), all in
-// nalgebra's per-element order.  b lives in LDS; one barrier per step.
-template <typename T>
-__global__ __launch_bounds__(1024) void getrs_kernel(const T *LU, int lda, int n, const int *ipiv, T *B, int ldb,
-                                                     int nrhs, int *info, int exact)
-{
-    extern __shared__ unsigned char smem_raw[];
-    T *b = reinterpret_cast<T *>(smem_raw);
-    __shared__ int fail;
-    const int t = threadIdx.x;
-    if (t == 0) fail = 0;
-    for (int c = 0; c < nrhs; ++c) {
-        T *bc = B + (size_t)c * ldb;
-        for (int r = t; r < n; r += blockDim.x) b[r] = bc[r];
-        __syncthreads();
-        if (t == 0) {
-            for (int i = 0; i < n; ++i) {
-                const int p = ipiv[i];
-                if (p != i) {
-                    const T v = b[i];
-                    b[i] = b[p];
-                    b[p] = v;
-                }
-            }
-        }
-        __syncthreads();
-        for (int i = 0; i + 1 < n; ++i) {
-            const T coeff = b[i];  // b_i / 1
-            for (int r = i + 1 + t; r < n; r += blockDim.x)
-                b[r] = sub_prod(b[r], coeff, LU[r + (size_t)i * lda], exact != 0);
-            __syncthreads();
-        }
-        for (int i = n - 1; i >= 0; --i) {
-            const T d = LU[i + (size_t)i * lda];
-            if (d == T(0)) {
-                if (t == 0 && fail == 0) fail = i + 1;
-                break;
-            }
-            const T coeff = b[i] / d;
-            __syncthreads();
-            if (t == 0) b[i] = coeff;
-            for (int r = t; r < i; r += blockDim.x)
-                b[r] = sub_prod(b[r], coeff, LU[r + (size_t)i * lda], exact != 0);
-            __syncthreads();
-        }
-        __syncthreads();
-        for (int r = t; r < n; r += blockDim.x) bc[r] = b[r];
-        __syncthreads();
-        if (fail) break;
-    }
-    if (t == 0 && info) *info = fail;
-}
-
 // ---------------------------------------------------------------- blocked Cholesky for n > 64
 // Rows below a factored 64-wide diagonal block: for each row r and panel
 // column j in order, a_rj = (a_rj - sum_{k<j} fl(L_jk * a_rk)) / L_jj with the
@@ -313,70 +258,6 @@ __global__ __launch_bounds__(64) void diag_det_kernel(const double *A, int lda, 
         out[0] = prod;
         out[1] = prod * prod;
         out[2] = lnsum;
-    }
-}
-
-// Cholesky solve for n > 64 on one workgroup: forward (solve.rs:488-519) and
-// backward with the 8-accumulator dotc order (solve.rs:697-755) or a tree sum.
-__global__ __launch_bounds__(256) void potrs_kernel(const double *L, int lda, int n, double *B, int ldb, int nrhs,
-                                                    int exact)
-{
-    extern __shared__ unsigned char smem_raw[];
-    double *b = reinterpret_cast<double *>(smem_raw);
-    __shared__ double part[256];
-    const int t = threadIdx.x;
-    for (int c = 0; c < nrhs; ++c) {
-        double *bc = B + (size_t)c * ldb;
-        for (int r = t; r < n; r += blockDim.x) b[r] = bc[r];
-        __syncthreads();
-        for (int i = 0; i < n; ++i) {
-            const double coeff = b[i] / L[i + (size_t)i * lda];
-            __syncthreads();
-            if (t == 0) b[i] = coeff;
-            for (int r = i + 1 + t; r < n; r += blockDim.x)
-                b[r] = sub_prod(b[r], coeff, L[r + (size_t)i * lda], exact != 0);
-            __syncthreads();
-        }
-        for (int i = n - 1; i >= 0; --i) {
-            const int len = n - i - 1;
-            const double *li = L + (i + 1) + (size_t)i * lda;
-            const double *bi = b + i + 1;
-            double dot = 0.0;
-            if (exact) {
-                if (t < 8) {
-                    const int full = len & ~7;
-                    double a = 0.0;
-                    for (int e = t; e < full; e += 8) a += li[e] * bi[e];
-                    part[t] = a;
-                }
-                __syncthreads();
-                if (t == 0) {
-                    const int full = len & ~7;
-                    double res = 0.0;
-                    res += part[0] + part[4];
-                    res += part[1] + part[5];
-                    res += part[2] + part[6];
-                    res += part[3] + part[7];
-                    for (int e = full; e < len; ++e) res += li[e] * bi[e];
-                    part[8] = res;
-                }
-            } else {
-                double a = 0.0;
-                for (int e = t; e < len; e += blockDim.x) a = fma(li[e], bi[e], a);
-                part[t] = a;
-                __syncthreads();
-                for (int s = 128; s > 0; s >>= 1) {
-                    if (t < s) part[t] += part[t + s];
-                    __syncthreads();
-                }
-                if (t == 0) part[8] = part[0];
-            }
-            __syncthreads();
-            if (t == 0) b[i] = (b[i] - part[8]) / L[i + (size_t)i * lda];
-            __syncthreads();
-        }
-        for (int r = t; r < n; r += blockDim.x) bc[r] = b[r];
-        __syncthreads();
     }
 }
 
@@ -533,17 +414,9 @@ int nrocm_dgetrs(nrocm_handle h, int n, int nrhs, const double *lu, int lda, con
     if (ldb < std::max(1, n)) return -8;
     if (!info) return -9;
     if (mode != NROCM_EXACT && mode != NROCM_FAST) return -10;
-    if (n >= NROCM_GETRS_LOOKBACK_MIN) {
-        // one workgroup per 64-row block, pipelined through published blocks
-        void *ws = nullptr;
-        const int s = nrocm_workspace(h, nrocm_getrs_scratch_bytes(n), &ws);
-        if (s != NROCM_OK) return s;
-        return nrocm_getrs_lookback(h, h->stream, n, nrhs, lu, lda, ipiv, b, ldb, info, mode == NROCM_EXACT, ws);
-    }
-    hipLaunchKernelGGL((getrs_kernel<double>), dim3(1), dim3(1024), (size_t)std::max(n, 1) * sizeof(double),
-                       h->stream, lu, lda, n, ipiv, b, ldb, nrhs, info, mode == NROCM_EXACT ? 1 : 0);
-    NROCM_CHECK_LAUNCH(h);
-    return NROCM_OK;
+    if (n >= NROCM_GETRS_LOOKBACK_MIN)
+        return nrocm_getrs_lookback(h, n, nrhs, lu, lda, ipiv, b, ldb, info, mode == NROCM_EXACT);
+    return nrocm_getrs_small(h, n, nrhs, lu, lda, ipiv, b, ldb, info, mode == NROCM_EXACT);
 }
 
 int nrocm_dpotrf(nrocm_handle h, int n, double *a, int lda, int *info, int mode)
@@ -593,16 +466,8 @@ int nrocm_dpotrs(nrocm_handle h, int n, int nrhs, const double *l, int lda, doub
     if (ldb < std::max(1, n)) return -7;
     if (mode != NROCM_EXACT && mode != NROCM_FAST) return -8;
     if (n == 0 || nrhs == 0) return NROCM_OK;
-    if (n >= NROCM_GETRS_LOOKBACK_MIN) {
-        void *ws = nullptr;
-        const int s = nrocm_workspace(h, nrocm_getrs_scratch_bytes(n), &ws);
-        if (s != NROCM_OK) return s;
-        return nrocm_potrs_lookback(h, h->stream, n, nrhs, l, lda, b, ldb, mode == NROCM_EXACT, ws);
-    }
-    hipLaunchKernelGGL(potrs_kernel, dim3(1), dim3(256), (size_t)n * sizeof(double), h->stream, l, lda, n, b, ldb,
-                       nrhs, mode == NROCM_EXACT ? 1 : 0);
-    NROCM_CHECK_LAUNCH(h);
-    return NROCM_OK;
+    if (n >= NROCM_GETRS_LOOKBACK_MIN) return nrocm_potrs_lookback(h, n, nrhs, l, lda, b, ldb, mode == NROCM_EXACT);
+    return nrocm_potrs_small(h, n, nrhs, l, lda, b, ldb, mode == NROCM_EXACT);
 }
 
 }  // extern "C"

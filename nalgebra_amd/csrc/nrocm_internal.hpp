@@ -5,6 +5,7 @@
 
 #include <cstdint>
 #include <cstdio>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -21,6 +22,24 @@ __device__ __forceinline__ void lds_barrier()
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+#endif
+
+#ifdef __HIPCC__
+constexpr size_t NROCM_LDS_BYTES = 160 * 1024;  // of one CU (gfx950), static and dynamic together
+
+// Lets kernel K be launched with dynamic LDS beyond the runtime's default (all
+// that its static LDS leaves).
+template <auto K>
+void nrocm_allow_lds()
+{
+    static std::once_flag once;
+    std::call_once(once, [] {
+        hipFuncAttributes a;
+        if (hipFuncGetAttributes(&a, (const void *)K) == hipSuccess && a.sharedSizeBytes < NROCM_LDS_BYTES)
+            (void)hipFuncSetAttribute((const void *)K, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                      (int)(NROCM_LDS_BYTES - a.sharedSizeBytes));
+    });
 }
 #endif
 

@@ -190,37 +190,6 @@ __global__ void copy_cols_kernel(const double *B, int ldb, int n, int nrhs, doub
     if (e < (size_t)n * nrhs) B0[e] = B[(e % n) + (e / n) * (size_t)ldb];
 }
 
-// QR's upper solve (qr.rs:224-256) on the leading n x n block.
-__global__ __launch_bounds__(256) void rsolve_exact_kernel(const double *QR, int n, int lda, const double *diag,
-                                                           double *B, int ldb, int nrhs, int *info)
-{
-    __shared__ double coeff_s;
-    __shared__ int fail;
-    if (threadIdx.x == 0) fail = 0;
-    __syncthreads();
-    for (int c = 0; c < nrhs && !fail; ++c) {
-        double *b = B + (size_t)c * ldb;
-        for (int i = n - 1; i >= 0; --i) {
-            if (threadIdx.x == 0) {
-                const double d = fabs(diag[i]);
-                if (d == 0.0) {
-                    fail = i + 1;
-                } else {
-                    coeff_s = b[i] / d;
-                    b[i] = coeff_s;
-                }
-            }
-            __syncthreads();
-            if (fail) break;
-            const double coeff = coeff_s;
-            for (int r = threadIdx.x; r < i; r += blockDim.x)
-                b[r] = axcpy1<double>(-coeff, QR[r + (size_t)i * lda], 1.0, 1.0, b[r]);
-            __syncthreads();
-        }
-    }
-    if (threadIdx.x == 0 && info) *info = fail;
-}
-
 }  // namespace
 
 // ---------------------------------------------------------------- batched tall least squares
@@ -341,9 +310,7 @@ int nrocm_dqr_rsolve(nrocm_handle h, int n, const double *qr, int lda, const dou
     if (!b && n > 0 && nrhs > 0) return -7;
     if (ldb < std::max(1, n)) return -8;
     if (!info) return -9;
-    hipLaunchKernelGGL(rsolve_exact_kernel, dim3(1), dim3(256), 0, h->stream, qr, n, lda, diag, b, ldb, nrhs, info);
-    NROCM_CHECK_LAUNCH(h);
-    return NROCM_OK;
+    return nrocm_qr_rsolve(h, n, nrhs, qr, lda, diag, b, ldb, info);
 }
 
 }  // extern "C"
