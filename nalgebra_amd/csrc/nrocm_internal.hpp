@@ -54,6 +54,8 @@ struct nrocm_handle_s {
     // Growable scratch on the device, reused across calls (ordered on `stream`).
     void *ws = nullptr;
     size_t ws_bytes = 0;
+    hipStream_t ws_stream = nullptr;  // of the last call that took the workspace
+    hipEvent_t ws_ev = nullptr;       // orders a call on another stream after it
     // Small device-side scalars (counters, flags, norms).
     void *small = nullptr;          // 4 KiB: int[0] Cholesky block info, ints from NROCM_SMALL_PLAN: LU row plan
     // Streams for independent launches that may run side by side (created on

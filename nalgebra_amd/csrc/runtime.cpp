@@ -19,8 +19,31 @@ int nrocm_fail(nrocm_handle h, int status, const char *msg)
     return status;
 }
 
+// Work that used the workspace on another stream of this handle comes first.
+static int order_after_last_user(nrocm_handle h)
+{
+    const bool moved = h->ws && h->ws_stream != h->stream;
+    hipStreamCaptureStatus now = hipStreamCaptureStatusNone, then = hipStreamCaptureStatusNone;
+    if (moved) NROCM_CHECK_HIP(h, hipStreamIsCapturing(h->stream, &now));
+    if (moved && now == hipStreamCaptureStatusNone) {
+        // the stream of the last use may be gone, or be recording a graph
+        const bool known = hipStreamIsCapturing(h->ws_stream, &then) == hipSuccess && then == hipStreamCaptureStatusNone;
+        if (!h->ws_ev) NROCM_CHECK_HIP(h, hipEventCreateWithFlags(&h->ws_ev, hipEventDisableTiming));
+        if (known && hipEventRecord(h->ws_ev, h->ws_stream) == hipSuccess) {
+            NROCM_CHECK_HIP(h, hipStreamWaitEvent(h->stream, h->ws_ev, 0));
+        } else {
+            (void)hipGetLastError();
+            if (then == hipStreamCaptureStatusNone) NROCM_CHECK_HIP(h, hipDeviceSynchronize());
+        }
+    }
+    h->ws_stream = h->stream;
+    return NROCM_OK;
+}
+
 int nrocm_workspace(nrocm_handle h, size_t bytes, void **ptr)
 {
+    const int s = order_after_last_user(h);
+    if (s != NROCM_OK) return s;
     if (bytes > h->ws_bytes) {
         if (h->ws) {
             // Work already queued may still use the old buffer.
@@ -114,6 +137,7 @@ int nrocm_destroy(nrocm_handle h)
         if (h->join_ev[i]) (void)hipEventDestroy(h->join_ev[i]);
     }
     if (h->fork_ev) (void)hipEventDestroy(h->fork_ev);
+    if (h->ws_ev) (void)hipEventDestroy(h->ws_ev);
     if (h->ws) (void)hipFree(h->ws);
     if (h->small) (void)hipFree(h->small);
     delete h;
