@@ -1,20 +1,19 @@
-// Blocked LU with partial pivoting (nrocm_dgetrf), LU solve (nrocm_dgetrs),
-// and the single-matrix Cholesky entry points (nrocm_dpotrf / nrocm_dpotrs).
+// LU with partial pivoting (nrocm_dgetrf), the windowed variant of the mixed
+// solver, and the single-matrix Cholesky entry points (nrocm_dpotrf).
 //
-// getrf schedule (right-looking, outer panel width 64):
+// Up to WHOLE_ROWS rows the whole matrix is one pipeline of column groups
+// (lu_columns.hpp).  Above:
 //   for each 64-wide panel [j0, j0+nb):
-//     for each base block [b0, b0+w) of the panel:
-//       panel_kernel        one workgroup factors the block's columns (rows b0..m)
-//       laswp               the block's swaps on the other panel columns
-//       trsm + update       U12 and the rank-w update of the rest of the panel
-//     swap plan + apply     the panel's swaps, composed into one row plan,
-//                           on all columns outside it
-//     trsm                  U12 = L11^{-1} A12 for the trailing columns
-//     trailing update       A22 -= L21 * U12: EXACT = ordered unfused SIMT,
-//                           FAST = FP64 MFMA, float working copies: FP32 or BF16 MFMA
+//     lu_columns_kernel   the panel, as a pipeline of column groups
+//     swap_rows_kernel    its swaps on all other columns
+//     trsm                U12 = L11^{-1} A12 for the trailing columns
+//     trailing update     A22 -= L21 * U12: EXACT = ordered unfused SIMT,
+//                         FAST = FP64 MFMA, float working copies: FP32 or BF16 MFMA
+//   where the next panel's 64 columns are updated first and the next panel then
+//   runs beside the update of the rest.
 #include "gemm_kernels.hpp"
 #include "internal_launch.hpp"
-#include "lu_kernels.hpp"
+#include "lu_columns.hpp"
 
 #include <algorithm>
 
@@ -22,52 +21,93 @@ using namespace nrocm_lu;
 
 namespace {
 
-template <typename T>
-struct PanelCfg {
-    int rpt, w;
-};
+// Whole matrices of up to this many rows are one pipeline; above it every group
+// takes too long to catch up with all the earlier ones (EXACT, one pipeline
+// against 64-column panels: n = 700 1.19 and 1.42 ms, 1000 1.94 and 2.15, 1100
+// 2.97 and 2.51, 2048 8.2 and 5.3).
+constexpr int WHOLE_ROWS = 1024;
 
-// Rows per thread and width of the one-workgroup panel for `rows` rows.
+// Words of the pipeline's buffer for an m x n matrix: L columns and pivots,
+// after a header of one ticket per panel.
+constexpr size_t LU_HEADER_BYTES = 2048;
 template <typename T>
-PanelCfg<T> panel_cfg(int rows)
+size_t lu_buffer_bytes(int m, int n)
 {
-    int rpt = 1;
-    while (rpt * PANEL_THREADS < rows) rpt *= 2;
-    return {rpt, panel_width(rpt, (int)sizeof(T))};
+    const size_t mn = (size_t)std::min(m, n);
+    return LU_HEADER_BYTES + (mn * m + mn) * sizeof(typename ColWord<T>::U);
 }
 
-template <typename T, int RPT>
-hipError_t launch_panel_rpt(hipStream_t st, int w_cap, T *A, int lda, int m, int col0, int w, int *ipiv,
-                            int *info)
+template <typename T>
+struct LuBuffer {
+    typedef typename ColWord<T>::U U;
+    int *tickets;
+    U *V, *H;
+    int ldv;
+    size_t words;
+
+    LuBuffer(void *p, int m, int n)
+        : tickets((int *)p), V((U *)((char *)p + LU_HEADER_BYTES)), H(V + (size_t)std::min(m, n) * m), ldv(m),
+          words((size_t)std::min(m, n) * m + std::min(m, n))
+    {
+    }
+    hipError_t clear(hipStream_t st)
+    {
+        hipLaunchKernelGGL((fill_words_kernel<U>), dim3(std::min<size_t>(4096, nrocm_cdiv(words, 1024) + 4)), dim3(256),
+                           0, st, V, words, ColWord<T>::EMPTY, tickets, (int)(LU_HEADER_BYTES / sizeof(int)));
+        return hipGetLastError();
+    }
+};
+
+template <typename T, typename G>
+hipError_t lu_columns_group(hipStream_t st, T *A, int lda, int m, int c0, int ncols, int kend, int *ipiv, int *info,
+                            LuBuffer<T> &b, int ticket)
 {
-    constexpr int WMAX = panel_width(RPT, (int)sizeof(T));
-    (void)w_cap;
-    hipLaunchKernelGGL((panel_kernel<T, RPT, WMAX>), dim3(1), dim3(PANEL_THREADS), 0, st, A, lda, m, col0, w,
-                       ipiv, info);
+    hipLaunchKernelGGL((lu_columns_kernel<T, G>), dim3(nrocm_cdiv(ncols, G::W)), dim3(G::CT), 0, st, A, lda, m, c0,
+                       ncols, kend, ipiv, info, b.V + (size_t)c0 * b.ldv, b.ldv, b.H + c0, b.tickets + ticket);
     return hipGetLastError();
 }
 
-template <typename T>
-hipError_t launch_panel(hipStream_t st, int rpt, int wcap, T *A, int lda, int m, int col0, int w, int *ipiv,
-                        int *info)
+template <typename T, typename G>
+hipError_t lu_left_group(hipStream_t st, T *A, int lda, int m, int c0, int kend, const int *ipiv, LuBuffer<T> &b)
 {
-    switch (rpt) {
-    case 1: return launch_panel_rpt<T, 1>(st, wcap, A, lda, m, col0, w, ipiv, info);
-    case 2: return launch_panel_rpt<T, 2>(st, wcap, A, lda, m, col0, w, ipiv, info);
-    case 4: return launch_panel_rpt<T, 4>(st, wcap, A, lda, m, col0, w, ipiv, info);
-    case 8: return launch_panel_rpt<T, 8>(st, wcap, A, lda, m, col0, w, ipiv, info);
-    case 16: return launch_panel_rpt<T, 16>(st, wcap, A, lda, m, col0, w, ipiv, info);
-    case 32: return launch_panel_rpt<T, 32>(st, wcap, A, lda, m, col0, w, ipiv, info);
-    default: return hipErrorInvalidValue;
-    }
+    const int groups = (int)nrocm_cdiv(kend - c0, G::W);
+    if (groups > 1 && m > c0 + G::W)
+        hipLaunchKernelGGL((lu_left_kernel<T, G::W>), dim3(nrocm_cdiv(m - c0 - G::W, 256), groups - 1), dim3(256), 0,
+                           st, A, lda, m, c0, kend, ipiv, b.V + (size_t)c0 * b.ldv, b.ldv);
+    return hipGetLastError();
+}
+
+#define LU_BY_ROWS(FN, rows, ...)                                                                        \
+    ((rows) <= Group256::ROWS   ? FN<T, Group256>(__VA_ARGS__)                                           \
+     : (rows) <= Group512::ROWS ? FN<T, Group512>(__VA_ARGS__)                                           \
+     : (rows) <= Group1K::ROWS  ? FN<T, Group1K>(__VA_ARGS__)                                            \
+     : (rows) <= Group2K::ROWS  ? FN<T, Group2K>(__VA_ARGS__)                                            \
+     : (rows) <= Group4K::ROWS  ? FN<T, Group4K>(__VA_ARGS__)                                            \
+     : (rows) <= Group8K::ROWS  ? FN<T, Group8K>(__VA_ARGS__) : FN<T, Group16K>(__VA_ARGS__))
+
+// Factors columns [c0, c0 + ncols) (those below kend) and brings them up to date.
+template <typename T>
+hipError_t lu_columns(hipStream_t st, T *A, int lda, int m, int c0, int ncols, int kend, int *ipiv, int *info,
+                      LuBuffer<T> &b, int ticket)
+{
+    return LU_BY_ROWS(lu_columns_group, m - c0, st, A, lda, m, c0, ncols, kend, ipiv, info, b, ticket);
+}
+
+// The L columns of all but the range's last group, their rows in final order.
+template <typename T>
+hipError_t lu_left(hipStream_t st, T *A, int lda, int m, int c0, int kend, const int *ipiv, LuBuffer<T> &b)
+{
+    return LU_BY_ROWS(lu_left_group, m - c0, st, A, lda, m, c0, kend, ipiv, b);
 }
 
 template <typename T>
-hipError_t laswp(hipStream_t st, T *A, int lda, int c0, int c1, const int *ipiv, int k0, int k1)
+hipError_t swap_rows(hipStream_t st, T *A, int lda, int m, const int *ipiv, int k0, int cnt, int ca0, int ca1, int cb0,
+                     int cb1)
 {
-    if (c1 <= c0 || k1 <= k0) return hipSuccess;
-    hipLaunchKernelGGL((laswp_kernel<T>), dim3(nrocm_cdiv(c1 - c0, 256)), dim3(256), 0, st, A, lda, c0, c1, ipiv,
-                       k0, k1);
+    const int cols = std::max(ca1 - ca0, 0) + std::max(cb1 - cb0, 0);
+    if (cols > 0)
+        hipLaunchKernelGGL((swap_rows_kernel<T>), dim3(nrocm_cdiv(cols, PLAN_COLS)), dim3(512), 0, st, A, lda, m, ipiv,
+                           k0, cnt, ca0, ca1, cb0, cb1);
     return hipGetLastError();
 }
 
@@ -120,46 +160,42 @@ hipError_t trailing(hipStream_t st, NrocmTrailing trail, T *A, int lda, int r0, 
     } while (0)
 
 template <typename T>
-int getrf_impl(nrocm_handle h, hipStream_t st, int m, int n, T *A, int lda, int *ipiv, int *info,
-               NrocmTrailing trail)
+int getrf_whole(nrocm_handle h, hipStream_t st, int m, int n, T *A, int lda, int *ipiv, int *info, void *buf)
 {
-    hipLaunchKernelGGL(fill_int_kernel, dim3(1), dim3(64), 0, st, info, 1, 0);
-    LU_TRY(hipGetLastError());
+    LuBuffer<T> b(buf, m, n);
     const int mn = std::min(m, n);
-    if (mn == 0) return NROCM_OK;
-    if (m > 32 * PANEL_THREADS) return nrocm_fail(h, NROCM_ERR_UNSUPPORTED, "getrf: more than 16384 rows");
+    LU_TRY(b.clear(st));
+    LU_TRY(lu_columns<T>(st, A, lda, m, 0, n, mn, ipiv, info, b, 0));
+    LU_TRY(lu_left<T>(st, A, lda, m, 0, mn, ipiv, b));
+    return NROCM_OK;
+}
+
+template <typename T>
+int getrf_panels(nrocm_handle h, hipStream_t st, int m, int n, T *A, int lda, int *ipiv, int *info,
+                 NrocmTrailing trail, void *buf)
+{
+    LuBuffer<T> b(buf, m, n);
+    const int mn = std::min(m, n);
     const bool exact = trail == TRAIL_EXACT;
     constexpr int NB = 64;
+    LU_TRY(b.clear(st));
+    LU_TRY(lu_columns<T>(st, A, lda, m, 0, std::min(NB, mn), std::min(NB, mn), ipiv, info, b, 0));
     for (int j0 = 0; j0 < mn; j0 += NB) {
-        const int nb = std::min(NB, mn - j0);
-        const int j1 = j0 + nb;
-        for (int b0 = j0; b0 < j1;) {
-            const PanelCfg<T> cfg = panel_cfg<T>(m - b0);
-            const int w = std::min(cfg.w, j1 - b0);
-            LU_TRY(launch_panel<T>(st, cfg.rpt, cfg.w, A, lda, m, b0, w, ipiv, info));
-            // swaps for panel columns [j0, b0); swaps + U12 + rank-w update for
-            // [b0+w, j1) -- always in exact order (the panel is narrow)
-            const int ncols = (b0 - j0) + (j1 - b0 - w);
-            if (ncols > 0) {
-                hipLaunchKernelGGL((panel_cols_kernel<T>), dim3(ncols), dim3(256), 0, st, A, lda, m, b0, w, j0,
-                                   b0 + w, j1, ipiv, 1);
-                LU_TRY(hipGetLastError());
-            }
-            b0 += w;
+        const int nb = std::min(NB, mn - j0), j1 = j0 + nb;
+        LU_TRY(lu_left<T>(st, A, lda, m, j0, j1, ipiv, b));
+        LU_TRY(swap_rows<T>(st, A, lda, m, ipiv, j0, nb, 0, j0, j1, n));
+        if (j1 < n) LU_TRY(trsm<T>(st, A, lda, j0, nb, j1, n, exact));
+        const int j2 = j1 < mn ? std::min(mn, j1 + NB) : j1;  // the next panel
+        if (j2 > j1) {
+            LU_TRY(trailing<T>(st, trail, A, lda, j1, m, j1, j2, j0, nb));
+            const int s = nrocm_fork_on(h, st, 1);
+            if (s != NROCM_OK) return s;
+            LU_TRY(lu_columns<T>(h->aux[0], A, lda, m, j1, j2 - j1, j2, ipiv, info, b, j1 / NB));
         }
-        // the panel's swaps on every column outside it, through a composed row plan
-        if (j0 > 0 || j1 < n) {
-            int *plan = (int *)h->small + NROCM_SMALL_PLAN;
-            hipLaunchKernelGGL(swap_plan_kernel, dim3(1), dim3(64), 0, st, ipiv, j0, j1, plan);
-            LU_TRY(hipGetLastError());
-            const int ncol = j0 + (n - j1);
-            hipLaunchKernelGGL((apply_plan_kernel<T>), dim3(nrocm_cdiv(ncol, 2)), dim3(256), 0, st, A, lda, plan, 0,
-                               j0, j1, n);
-            LU_TRY(hipGetLastError());
-        }
-        if (j1 < n) {
-            LU_TRY(trsm<T>(st, A, lda, j0, nb, j1, n, exact));
-            LU_TRY(trailing<T>(st, trail, A, lda, j1, m, j1, n, j0, nb));
+        LU_TRY(trailing<T>(st, trail, A, lda, j1, m, j2, n, j0, nb));
+        if (j2 > j1) {
+            const int s = nrocm_join_on(h, st, 1);
+            if (s != NROCM_OK) return s;
         }
     }
     return NROCM_OK;
@@ -333,16 +369,29 @@ int getrf_window_impl(nrocm_handle h, hipStream_t st, int n, T *A, int lda, int 
 
 // ---------------------------------------------------------------- internal entry points
 
-// The blocked factorisation is thousands of small launches at large n, so the
-// sequence is captured once per (shape, buffers, flavour) and replayed.
+// Above WHOLE_ROWS rows the factorisation is some hundred launches on two
+// streams, captured once per (shape, buffers, flavour) and replayed.
 template <typename T>
 int getrf_graph(nrocm_handle h, int m, int n, T *A, int lda, int *ipiv, int *info, NrocmTrailing trail)
 {
-    if (std::min(m, n) <= 64) return getrf_impl<T>(h, h->stream, m, n, A, lda, ipiv, info, trail);
-    const long long key[8] = {1000 + (long long)sizeof(T), m, n, lda, (long long)A, (long long)ipiv,
-                              (long long)info, (long long)trail};
+    if (std::min(m, n) == 0) {
+        hipLaunchKernelGGL(fill_int_kernel, dim3(1), dim3(64), 0, h->stream, info, 1, 0);
+        NROCM_CHECK_LAUNCH(h);
+        return NROCM_OK;
+    }
+    if (m > COLUMNS_ROWS_MAX) return nrocm_fail(h, NROCM_ERR_UNSUPPORTED, "getrf: more than 16384 rows");
+    void *buf = nullptr;
+    int s = nrocm_workspace(h, lu_buffer_bytes<T>(m, n), &buf, NROCM_WS_LU);
+    if (s != NROCM_OK) return s;
+    hipLaunchKernelGGL(fill_int_kernel, dim3(1), dim3(64), 0, h->stream, info, 1, 0);
+    NROCM_CHECK_LAUNCH(h);
+    if (m <= WHOLE_ROWS || std::min(m, n) <= 64) return getrf_whole<T>(h, h->stream, m, n, A, lda, ipiv, info, buf);
+    s = nrocm_aux_init(h);  // streams and events exist before the capture
+    if (s != NROCM_OK) return s;
+    const long long key[8] = {1000 + (long long)sizeof(T) + 16 * (long long)trail, (long long)m << 32 | n, lda,
+                              (long long)A, (long long)ipiv, (long long)info, (long long)buf, 0};
     return nrocm_graph_run(h, key, [&](hipStream_t st) {
-        return getrf_impl<T>(h, st, m, n, A, lda, ipiv, info, trail);
+        return getrf_panels<T>(h, st, m, n, A, lda, ipiv, info, trail, buf);
     });
 }
 

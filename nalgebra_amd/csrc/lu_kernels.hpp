@@ -15,27 +15,6 @@
 
 namespace nrocm_lu {
 
-// Two wavefronts per SIMD (up to 256 VGPRs per thread); the per-column
-// barrier synchronises eight wavefronts.
-constexpr int PANEL_THREADS = 512;
-
-// Panel width per rows-per-thread: RPT * W values of the panel plus the W
-// values of the pivot row stay in registers without spilling.
-__host__ __device__ constexpr int panel_width(int rpt, int elem_bytes)
-{
-    return elem_bytes == 8 ? (rpt <= 1 ? 32 : rpt == 2 ? 16 : rpt == 4 ? 8 : rpt == 8 ? 4 : rpt == 16 ? 2 : 1)
-                           : (rpt <= 2 ? 32 : rpt == 4 ? 16 : rpt == 8 ? 8 : rpt == 16 ? 4 : 2);
-}
-
-// a beats b under icamax's rule (src/base/min_max.rs:221-241): larger |x|,
-// ties to the lower index.  NaN never wins except at the column head, which
-// the caller encodes as +inf with the lowest index.
-template <typename V>
-__device__ __forceinline__ bool beats_v(V av, int ai, V bv, int bi)
-{
-    return av > bv || (av == bv && ai < bi);
-}
-
 // 32-bit DPP move with `old` kept where the source lane is outside the pattern.
 template <int CTRL, int ROWMASK>
 __device__ __forceinline__ int dpp32(int old, int v)
@@ -58,32 +37,50 @@ __device__ __forceinline__ float dpp_f32(float old, float v)
     return __int_as_float(dpp32<CTRL, ROWMASK>(__float_as_int(old), __float_as_int(v)));
 }
 
-template <typename V, int CTRL, int ROWMASK>
-__device__ __forceinline__ void argmax_dpp_step(V &bv, int &bi)
+// one instruction: fmax would first quiet NaNs, of which there are none here
+__device__ __forceinline__ double max_dpp(double v, double o)
 {
-    V ov;
-    if constexpr (sizeof(V) == 8) ov = dpp_f64<CTRL, ROWMASK>(V(-1), bv);
-    else ov = dpp_f32<CTRL, ROWMASK>(V(-1), bv);
-    const int oi = dpp32<CTRL, ROWMASK>(0x7fffffff, bi);
-    if (beats_v(ov, oi, bv, bi)) {
-        bv = ov;
-        bi = oi;
-    }
+    double r;
+    asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(v), "v"(o));
+    return r;
+}
+__device__ __forceinline__ float max_dpp(float v, float o)
+{
+    float r;
+    asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(v), "v"(o));
+    return r;
+}
+template <int CTRL, int ROWMASK>
+__device__ __forceinline__ double dpp_value(double v) { return dpp_f64<CTRL, ROWMASK>(-1.0, v); }
+template <int CTRL, int ROWMASK>
+__device__ __forceinline__ float dpp_value(float v) { return dpp_f32<CTRL, ROWMASK>(-1.0f, v); }
+
+// Wavefront maximum of non-NaN values >= -1; lane 63 ends with it.  Row scans by
+// row_shr 1, 2, 4, 8, then row_bcast 15 into rows 1 and 3 and row_bcast 31 into
+// rows 2 and 3.
+template <typename V>
+__device__ __forceinline__ V max_wave(V v)
+{
+    v = max_dpp(v, dpp_value<0x111, 0xf>(v));
+    v = max_dpp(v, dpp_value<0x112, 0xf>(v));
+    v = max_dpp(v, dpp_value<0x114, 0xf>(v));
+    v = max_dpp(v, dpp_value<0x118, 0xf>(v));
+    v = max_dpp(v, dpp_value<0x142, 0xa>(v));
+    v = max_dpp(v, dpp_value<0x143, 0xc>(v));
+    return v;
 }
 
-// Wavefront argmax under the first-index strict-max rule; lane 63 ends with
-// the result.  Row scans by row_shr 1, 2, 4, 8, then row_bcast 15 into rows 1
-// and 3 and row_bcast 31 into rows 2 and 3.  The rule is a total order on
-// (value, row) pairs, so the combination order does not change the winner.
-template <typename V>
-__device__ __forceinline__ void argmax_wave(V &bv, int &bi)
+// Wavefront minimum of int positions; lane 63 ends with it.
+__device__ __forceinline__ int min_wave(int p)
 {
-    argmax_dpp_step<V, 0x111, 0xf>(bv, bi);
-    argmax_dpp_step<V, 0x112, 0xf>(bv, bi);
-    argmax_dpp_step<V, 0x114, 0xf>(bv, bi);
-    argmax_dpp_step<V, 0x118, 0xf>(bv, bi);
-    argmax_dpp_step<V, 0x142, 0xa>(bv, bi);
-    argmax_dpp_step<V, 0x143, 0xc>(bv, bi);
+    constexpr int M = 0x7fffffff;
+    p = min(p, dpp32<0x111, 0xf>(M, p));
+    p = min(p, dpp32<0x112, 0xf>(M, p));
+    p = min(p, dpp32<0x114, 0xf>(M, p));
+    p = min(p, dpp32<0x118, 0xf>(M, p));
+    p = min(p, dpp32<0x142, 0xa>(M, p));
+    p = min(p, dpp32<0x143, 0xc>(M, p));
+    return p;
 }
 
 // Returns v unchanged.  Copy loops whose values pass through this are not
@@ -114,145 +111,6 @@ __device__ __forceinline__ T sub_prod(T acc, T x, T y, bool exact)
         }
     }
     return fma(-x, y, acc);
-}
-
-// Unblocked LU of the panel A[row0.., col0..col0+w) held in registers by one
-// PANEL_THREADS-thread workgroup; thread t holds rows row0 + t + PANEL_THREADS*s, s < RPT.
-// Pivot rows are recorded as global row indices in ipiv[col0 + c].
-template <typename T, int RPT, int W>
-__global__ __launch_bounds__(PANEL_THREADS) void panel_kernel(T *A, int lda, int m, int col0, int w,
-                                                              int *ipiv, int *info)
-{
-    __shared__ T red_v[PANEL_THREADS / 64];
-    __shared__ int red_i[PANEL_THREADS / 64];
-    __shared__ T rowbuf[2][2][W];  // [parity][0: pivot row, 1: row i]
-    const int t = threadIdx.x;
-    const int lane = t & 63, wv = t >> 6;
-    const int row0 = col0;
-
-    T x[RPT][W];
-#pragma unroll
-    for (int s = 0; s < RPT; ++s) {
-        const int r = row0 + t + PANEL_THREADS * s;
-#pragma unroll
-        for (int c = 0; c < W; ++c) x[s][c] = (r < m && c < w) ? A[r + (size_t)(col0 + c) * lda] : T(0);
-    }
-
-    // No break/continue in this loop: it must unroll completely so that x
-    // stays in registers.
-#pragma unroll
-    for (int c = 0; c < W; ++c) {
-        if (c < w) {
-            const int i = row0 + c;  // pivot row position (global)
-            // ---- pivot search over rows i..m-1 of column c
-            T bv = T(-1);
-            int bi = 0x7fffffff;
-#pragma unroll
-            for (int s = 0; s < RPT; ++s) {
-                const int r = row0 + t + PANEL_THREADS * s;
-                T v = fabs(x[s][c]);
-                v = (v != v) ? ((r == i) ? T(__builtin_inf()) : T(-1)) : v;  // NaN rule
-                v = (r >= i && r < m) ? v : T(-1);
-                // a thread visits its rows in increasing order: a tie keeps the lower row
-                if (v > bv) { bv = v; bi = r; }
-            }
-            argmax_wave<T>(bv, bi);
-            if (lane == 63) { red_v[wv] = bv; red_i[wv] = bi; }
-            lds_barrier();
-            bv = red_v[0];
-            bi = red_i[0];
-#pragma unroll
-            for (int q = 1; q < PANEL_THREADS / 64; ++q)
-                if (beats_v(red_v[q], red_i[q], bv, bi)) { bv = red_v[q]; bi = red_i[q]; }
-            const int piv = bi;
-            // ---- exchange rows i and piv through LDS (only their owners copy)
-            T(*rb)[W] = rowbuf[c & 1];
-            const int opiv = piv - row0 - t, oi = i - row0 - t;  // multiples of PANEL_THREADS for the owners
-            if (opiv >= 0 && opiv % PANEL_THREADS == 0) {
-#pragma unroll
-                for (int s = 0; s < RPT; ++s)
-                    if (opiv == PANEL_THREADS * s) {
-#pragma unroll
-                        for (int q = 0; q < W; ++q) rb[0][q] = pass(x[s][q]);
-                    }
-            }
-            if (oi >= 0 && oi % PANEL_THREADS == 0) {
-#pragma unroll
-                for (int s = 0; s < RPT; ++s)
-                    if (oi == PANEL_THREADS * s) {
-#pragma unroll
-                        for (int q = 0; q < W; ++q) rb[1][q] = pass(x[s][q]);
-                    }
-            }
-            lds_barrier();
-            const T d = rb[0][c];  // the pivot value
-            if (t == 0) ipiv[col0 + c] = (d == T(0)) ? i : piv;
-            if (d == T(0)) {
-                // lu.rs:107-110: all-zero column, nothing is swapped or updated
-                if (t == 0 && info && *info == 0) *info = i + 1;
-            } else {
-                const T inv = T(1) / d;
-                // rows i and piv trade places (their owners only)
-                if (oi >= 0 && oi % PANEL_THREADS == 0) {
-#pragma unroll
-                    for (int s = 0; s < RPT; ++s)
-                        if (oi == PANEL_THREADS * s) {
-#pragma unroll
-                            for (int q = 0; q < W; ++q) x[s][q] = pass(rb[0][q]);
-                        }
-                }
-                if (piv != i && opiv >= 0 && opiv % PANEL_THREADS == 0) {
-#pragma unroll
-                    for (int s = 0; s < RPT; ++s)
-                        if (opiv == PANEL_THREADS * s) {
-#pragma unroll
-                            for (int q = 0; q < W; ++q) x[s][q] = pass(rb[1][q]);
-                        }
-                }
-#pragma unroll
-                for (int s = 0; s < RPT; ++s) {
-                    const int r = row0 + t + PANEL_THREADS * s;
-                    if (r > i && r < m) {
-                        const T l = x[s][c] * inv;
-                        x[s][c] = l;
-#pragma unroll
-                        for (int q = 0; q < W; ++q)  // constant trip count: unrolls before c does
-                            if (q > c) x[s][q] = sub_prod(x[s][q], rb[0][q], l, true);
-                    }
-                }
-            }
-        }
-    }
-    // A copy of t the compiler cannot see through, so the load addresses and
-    // row predicates are recomputed here instead of living in registers.
-    int tt = t;
-    asm volatile("" : "+v"(tt));
-#pragma unroll
-    for (int s = 0; s < RPT; ++s) {
-        const int r = row0 + tt + PANEL_THREADS * s;
-        if (r < m) {
-#pragma unroll
-            for (int c = 0; c < W; ++c)
-                if (c < w) A[r + (size_t)(col0 + c) * lda] = x[s][c];
-        }
-    }
-}
-
-// Row swaps ipiv[k0..k1) applied in order to columns [c0, c1) (one thread per column).
-template <typename T>
-__global__ void laswp_kernel(T *A, int lda, int c0, int c1, const int *ipiv, int k0, int k1)
-{
-    const int c = c0 + blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= c1) return;
-    T *col = A + (size_t)c * lda;
-    for (int i = k0; i < k1; ++i) {
-        const int p = ipiv[i];
-        if (p != i) {
-            const T a = col[i];
-            col[i] = col[p];
-            col[p] = a;
-        }
-    }
 }
 
 // U12 = L11^{-1} A12 for a unit-lower L11 (k x k, k <= 64) at A[r0, r0] and the
@@ -347,149 +205,10 @@ __global__ __launch_bounds__(256) void update_kernel(T *C, int ldc, int m, int n
         }
 }
 
-// For each column c of [c0, c1) (one workgroup each) after the base block
-// [b0, b0+w) has been factored: apply its w row swaps to the column; when
-// c >= b0 + w also form U12 (rows b0..b0+w, unit-lower solve with L11) and
-// apply the rank-w update to rows b0+w..m.  Every element's terms are applied
-// in increasing k (EXACT: fl(a - fl(u*l))), as nalgebra's gauss steps do.
-template <typename T>
-__global__ __launch_bounds__(256) void panel_cols_kernel(T *A, int lda, int m, int b0, int w, int cl, int cr0,
-                                                         int cr1, const int *ipiv, int exact)
-{
-    __shared__ int pos[64];      // touched row positions
-    __shared__ int who[64];      // original position whose value ends at pos[q]
-    __shared__ int piv[32];
-    __shared__ int nt;
-    __shared__ T L11[32][33];
-    __shared__ T U[32];
-    const int t = threadIdx.x;
-    const int idx = blockIdx.x;
-    // columns [cl, b0) swap only; columns [cr0, cr1) swap + solve + update
-    const int c = idx < b0 - cl ? cl + idx : cr0 + (idx - (b0 - cl));
-    const bool full = c >= cr0;
-    T *col = A + (size_t)c * lda;
-    if (t < w) piv[t] = ipiv[b0 + t];
-    if (full)
-        for (int e = t; e < w * w; e += blockDim.x)
-            L11[e % w][e / w] = A[(b0 + e % w) + (size_t)(b0 + e / w) * lda];
-    __syncthreads();
-    // compose the w swaps on indices only
-    if (t == 0) {
-        int n_ = 0;
-        for (int i = 0; i < w; ++i) {
-            const int p = piv[i];
-            int a = -1, b = -1;
-            for (int q = 0; q < n_; ++q) {
-                if (pos[q] == b0 + i) a = q;
-                if (pos[q] == p) b = q;
-            }
-            if (a < 0) { a = n_; pos[n_] = b0 + i; who[n_] = b0 + i; ++n_; }
-            if (b < 0) { b = n_; pos[n_] = p; who[n_] = p; ++n_; }
-            const int tw = who[a];
-            who[a] = who[b];
-            who[b] = tw;
-        }
-        nt = n_;
-    }
-    __syncthreads();
-    T v = T(0);
-    if (t < nt) v = col[who[t]];
-    __syncthreads();
-    if (t < nt) col[pos[t]] = v;
-    __syncthreads();
-    if (!full) return;
-    // U12 for this column: rows b0..b0+w, unit lower L11 (one wavefront)
-    if (t < 64) {
-        T u = t < w ? col[b0 + t] : T(0);
-        for (int i = 0; i < w - 1; ++i) {
-            const T ui = __shfl(u, i);
-            if (t > i && t < w) u = sub_prod(u, ui, L11[t][i], exact != 0);
-        }
-        if (t < w) {
-            col[b0 + t] = u;
-            U[t] = u;
-        }
-    }
-    __syncthreads();
-    // rank-w update of rows b0+w..m, terms in increasing k; RU rows per
-    // thread have their loads in flight together
-    constexpr int RU = 8;
-    for (int rb = b0 + w + t; rb < m; rb += 256 * RU) {
-        T a[RU];
-#pragma unroll
-        for (int u = 0; u < RU; ++u) {
-            const int r = rb + 256 * u;
-            a[u] = r < m ? col[r] : T(0);
-        }
-        for (int q = 0; q < w; ++q) {
-            const T uq = U[q];
-            const T *Lq = A + (size_t)(b0 + q) * lda;
-            T l[RU];
-#pragma unroll
-            for (int u = 0; u < RU; ++u) {
-                const int r = rb + 256 * u;
-                l[u] = r < m ? Lq[r] : T(0);
-            }
-#pragma unroll
-            for (int u = 0; u < RU; ++u) a[u] = sub_prod(a[u], uq, l[u], exact != 0);
-        }
-#pragma unroll
-        for (int u = 0; u < RU; ++u) {
-            const int r = rb + 256 * u;
-            if (r < m) col[r] = a[u];
-        }
-    }
-}
-
-// Composition of the row swaps ipiv[k0..k1) (k1 - k0 <= 64, applied in
-// order, as LU::new swaps whole rows at every step) into a row plan:
-// plan[0] = number nt of touched positions; after the swaps, position
-// plan[1 + s] holds the value that was at position plan[1 + PLAN_MAX + s].
+// Row plan of a window's permutation: plan[0] = number nt of touched
+// positions; afterwards position plan[1 + s] holds the value that was at
+// position plan[1 + PLAN_MAX + s].
 constexpr int PLAN_MAX = 128;
-
-// One wavefront; lane l keeps slots l and l + 64 of the plan in registers, and
-// the slots of positions i and p are found by ballot, so no barriers are needed.
-__global__ __launch_bounds__(64) void swap_plan_kernel(const int *ipiv, int k0, int k1, int *plan)
-{
-    const int l = threadIdx.x;
-    int pos0 = -1, who0 = -1, pos1 = -1, who1 = -1;
-    const int myp = (l < k1 - k0) ? ipiv[k0 + l] : 0;
-    int cnt = 0;
-    for (int i = k0; i < k1; ++i) {
-        const int p = __shfl(myp, i - k0);
-        if (p == i) continue;  // uniform: no swap at this step
-        const unsigned long long ma0 = __ballot(pos0 == i), ma1 = __ballot(pos1 == i);
-        const unsigned long long mb0 = __ballot(pos0 == p), mb1 = __ballot(pos1 == p);
-        int a = ma0 ? __builtin_ctzll(ma0) : ma1 ? 64 + __builtin_ctzll(ma1) : -1;
-        int b = mb0 ? __builtin_ctzll(mb0) : mb1 ? 64 + __builtin_ctzll(mb1) : -1;
-        if (a < 0) {
-            a = cnt++;
-            if (l == (a & 63)) {
-                if (a < 64) { pos0 = i; who0 = i; } else { pos1 = i; who1 = i; }
-            }
-        }
-        if (b < 0) {
-            b = cnt++;
-            if (l == (b & 63)) {
-                if (b < 64) { pos0 = p; who0 = p; } else { pos1 = p; who1 = p; }
-            }
-        }
-        // swap who[a] and who[b]
-        const int wa = __shfl(a < 64 ? who0 : who1, a & 63);
-        const int wb = __shfl(b < 64 ? who0 : who1, b & 63);
-        if (l == (a & 63)) { if (a < 64) who0 = wb; else who1 = wb; }
-        if (l == (b & 63)) { if (b < 64) who0 = wa; else who1 = wa; }
-    }
-    if (l == 0) plan[0] = cnt;
-    if (l < cnt) {
-        plan[1 + l] = pos0;
-        plan[1 + PLAN_MAX + l] = who0;
-    }
-    if (64 + l < cnt) {
-        plan[1 + 64 + l] = pos1;
-        plan[1 + PLAN_MAX + 64 + l] = who1;
-    }
-}
 
 // Applies a row plan to the columns [ca0, ca1) and [cb0, cb1): two columns
 // per workgroup, one thread per touched position; every value is read before

@@ -52,10 +52,15 @@ struct nrocm_handle_s {
     std::string last_error;
 
     // Growable scratch on the device, reused across calls (ordered on `stream`).
-    void *ws = nullptr;
-    size_t ws_bytes = 0;
-    hipStream_t ws_stream = nullptr;  // of the last call that took the workspace
-    hipEvent_t ws_ev = nullptr;       // orders a call on another stream after it
+    struct Scratch {
+        void *ptr = nullptr;
+        size_t bytes = 0;
+        hipStream_t stream = nullptr;  // of the last call that took it
+        bool captured = false;         // a caller's graph holds its address
+    };
+    Scratch ws[2];                  // NROCM_WS_MAIN, NROCM_WS_LU
+    hipEvent_t ws_ev = nullptr;     // orders a call on another stream after the last
+    std::vector<void *> retired;    // outgrown scratch that a caller's graph may still use
     // Small device-side scalars (counters, flags, norms).
     void *small = nullptr;          // 4 KiB: int[0] Cholesky block info, ints from NROCM_SMALL_PLAN: LU row plan
     // Streams for independent launches that may run side by side (created on
@@ -119,8 +124,14 @@ struct nrocm_batch_s {
 // Records a message on the handle and returns NROCM_ERR_HIP.
 int nrocm_fail_hip(nrocm_handle h, hipError_t e, const char *what);
 int nrocm_fail(nrocm_handle h, int status, const char *msg);
-// Ensures at least `bytes` of workspace; synchronises the stream when it grows.
-int nrocm_workspace(nrocm_handle h, size_t bytes, void **ptr);
+// Ensures at least `bytes` of scratch; synchronises the stream when it grows.
+// NROCM_WS_LU is the LU's own (other routines factor while they hold the main
+// one); it starts with NROCM_WS_LU_FIRST bytes, all that min(m, n) <= 64 needs.
+// On a stream under capture nothing is freed, and what the graph may hold stays
+// until the handle is destroyed.
+enum { NROCM_WS_MAIN = 0, NROCM_WS_LU = 1 };
+constexpr size_t NROCM_WS_LU_FIRST = (size_t)16384 * 64 * 8 + 8192;
+int nrocm_workspace(nrocm_handle h, size_t bytes, void **ptr, int which = NROCM_WS_MAIN);
 // Forks the handle's auxiliary streams from its stream (nrocm_fork) and joins
 // them back (nrocm_join): work launched on aux[i] in between runs concurrently
 // with the other auxiliary streams and after everything queued before the fork.

@@ -467,6 +467,12 @@ __global__ __launch_bounds__(PT) void geqrf_columns_kernel(T *A, int m, int n, i
         for (int s = 0; s < RPT; ++s) w[s] = nw[s];
         hw = nh;
     }
+    // every column has arrived on every path: else its first use after the first
+    // published axis would wait for those stores
+#pragma unroll
+    for (int c = 0; c < PC; ++c)
+#pragma unroll
+        for (int s = 0; s < RPT; ++s) asm volatile("" : "+v"(x[c][s]));
     own_columns<T, RPT, PC, 0>(x, c0, nc, m, mn, prod, sc, fac, diag, V, H);
 #pragma unroll
     for (int c = 0; c < PC; ++c)

@@ -19,47 +19,69 @@ int nrocm_fail(nrocm_handle h, int status, const char *msg)
     return status;
 }
 
-// Work that used the workspace on another stream of this handle comes first.
-static int order_after_last_user(nrocm_handle h)
+// Work that used the scratch on another stream of this handle comes first.
+static int order_after_last_user(nrocm_handle h, nrocm_handle_s::Scratch &w)
 {
-    const bool moved = h->ws && h->ws_stream != h->stream;
-    hipStreamCaptureStatus now = hipStreamCaptureStatusNone, then = hipStreamCaptureStatusNone;
-    if (moved) NROCM_CHECK_HIP(h, hipStreamIsCapturing(h->stream, &now));
-    if (moved && now == hipStreamCaptureStatusNone) {
+    if (w.ptr && w.stream != h->stream) {
         // the stream of the last use may be gone, or be recording a graph
-        const bool known = hipStreamIsCapturing(h->ws_stream, &then) == hipSuccess && then == hipStreamCaptureStatusNone;
+        hipStreamCaptureStatus then = hipStreamCaptureStatusNone;
+        const bool known = hipStreamIsCapturing(w.stream, &then) == hipSuccess && then == hipStreamCaptureStatusNone;
         if (!h->ws_ev) NROCM_CHECK_HIP(h, hipEventCreateWithFlags(&h->ws_ev, hipEventDisableTiming));
-        if (known && hipEventRecord(h->ws_ev, h->ws_stream) == hipSuccess) {
+        if (known && hipEventRecord(h->ws_ev, w.stream) == hipSuccess) {
             NROCM_CHECK_HIP(h, hipStreamWaitEvent(h->stream, h->ws_ev, 0));
         } else {
             (void)hipGetLastError();
             if (then == hipStreamCaptureStatusNone) NROCM_CHECK_HIP(h, hipDeviceSynchronize());
         }
     }
-    h->ws_stream = h->stream;
     return NROCM_OK;
 }
 
-int nrocm_workspace(nrocm_handle h, size_t bytes, void **ptr)
+int nrocm_workspace(nrocm_handle h, size_t bytes, void **ptr, int which)
 {
-    const int s = order_after_last_user(h);
-    if (s != NROCM_OK) return s;
-    if (bytes > h->ws_bytes) {
-        if (h->ws) {
-            // Work already queued may still use the old buffer.
-            NROCM_CHECK_HIP(h, hipStreamSynchronize(h->stream));
-            NROCM_CHECK_HIP(h, hipFree(h->ws));
-            h->ws = nullptr;
-            h->ws_bytes = 0;
-        }
-        size_t want = bytes + bytes / 4;
-        if (hipMalloc(&h->ws, want) != hipSuccess) {
-            h->ws = nullptr;
-            return nrocm_fail(h, NROCM_ERR_ALLOC, "workspace allocation failed");
-        }
-        h->ws_bytes = want;
+    nrocm_handle_s::Scratch &w = h->ws[which];
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(h->stream, &cap) != hipSuccess) {
+        (void)hipGetLastError();  // the legacy stream beside a capture
+        cap = hipStreamCaptureStatusActive;
     }
-    *ptr = h->ws;
+    const bool capturing = cap != hipStreamCaptureStatusNone;
+    if (!capturing) {
+        const int s = order_after_last_user(h, w);
+        if (s != NROCM_OK) return s;
+    }
+    if (bytes > w.bytes) {
+        // an allocation is no part of a capture, but is not allowed beside one
+        // unless the thread says so
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        if (capturing) NROCM_CHECK_HIP(h, hipThreadExchangeStreamCaptureMode(&mode));
+        int status = NROCM_OK;
+        if (w.ptr) {
+            if (capturing || w.captured) {
+                h->retired.push_back(w.ptr);
+            } else {
+                // Work already queued may still use the old buffer.
+                hipError_t e = hipStreamSynchronize(h->stream);
+                if (e == hipSuccess) e = hipFree(w.ptr);
+                if (e != hipSuccess) status = nrocm_fail_hip(h, e, "workspace release");
+            }
+            if (status == NROCM_OK) w = nrocm_handle_s::Scratch();
+        }
+        const size_t want = bytes + bytes / 4;
+        if (status == NROCM_OK) {
+            if (hipMalloc(&w.ptr, want) == hipSuccess) {
+                w.bytes = want;
+            } else {
+                w.ptr = nullptr;
+                status = nrocm_fail(h, NROCM_ERR_ALLOC, "workspace allocation failed");
+            }
+        }
+        if (capturing) (void)hipThreadExchangeStreamCaptureMode(&mode);
+        if (status != NROCM_OK) return status;
+    }
+    w.captured = w.captured || capturing;
+    w.stream = h->stream;
+    *ptr = w.ptr;
     return NROCM_OK;
 }
 
@@ -119,6 +141,13 @@ int nrocm_create(nrocm_handle *handle)
         delete h;
         return NROCM_ERR_ALLOC;
     }
+    nrocm_handle_s::Scratch &lu = h->ws[NROCM_WS_LU];
+    if (hipMalloc(&lu.ptr, NROCM_WS_LU_FIRST) != hipSuccess) {
+        (void)hipFree(h->small);
+        delete h;
+        return NROCM_ERR_ALLOC;
+    }
+    lu.bytes = NROCM_WS_LU_FIRST;
     *handle = h;
     return NROCM_OK;
 }
@@ -138,7 +167,9 @@ int nrocm_destroy(nrocm_handle h)
     }
     if (h->fork_ev) (void)hipEventDestroy(h->fork_ev);
     if (h->ws_ev) (void)hipEventDestroy(h->ws_ev);
-    if (h->ws) (void)hipFree(h->ws);
+    for (auto &w : h->ws)
+        if (w.ptr) (void)hipFree(w.ptr);
+    for (void *p : h->retired) (void)hipFree(p);
     if (h->small) (void)hipFree(h->small);
     delete h;
     return NROCM_OK;
