@@ -167,8 +167,9 @@ using GemmMedium = GemmShape<64, 64, 2, 1, 32>;   // wavefront 32 x 32
 using GemmSmall = GemmShape<32, 32, 1, 4, 64>;    // 4 k-groups of one 32 x 32 block
 
 template <typename TS> struct Vec16;
-template <> struct Vec16<double> { typedef double T __attribute__((ext_vector_type(2))); static constexpr int N = 2; };
-template <> struct Vec16<float> { typedef float T __attribute__((ext_vector_type(4))); static constexpr int N = 4; };
+// (aligned as its elements: for loads from any leading dimension)
+template <> struct Vec16<double> { typedef double T __attribute__((ext_vector_type(2), aligned(8))); static constexpr int N = 2; };
+template <> struct Vec16<float> { typedef float T __attribute__((ext_vector_type(4), aligned(4))); static constexpr int N = 4; };
 
 // wavefronts per SIMD the register allocation is held to: two for the FP64
 // 128 x 128 shape (its 64 accumulator doubles per lane fit beside the operand
@@ -183,13 +184,14 @@ constexpr int gemm_waves()
 template <typename TS, int MODE, typename SH>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(gemm_waves<TS, SH>()))) void gemm_cm_kernel(int m, int n, int k, TS alpha, const TS *__restrict__ A,
                                                       long lda, const TS *__restrict__ B, long ldb, TS beta,
-                                                      TS *__restrict__ C, long ldc, int vec_ok)
+                                                      TS *__restrict__ C, long ldc)
 {
     static_assert(MODE == MODE_F64 || MODE == MODE_F32, "column-major GEMM: FP64 or FP32 MFMA");
     constexpr int BM = SH::BM, BN = SH::BN, BK = SH::BK, KSPLIT = SH::KSPLIT;
     constexpr int WGM = SH::WGM, FM = SH::FM, FN = SH::FN;
     using AccT = typename Acc<MODE>::T;
     using V = typename Vec16<TS>::T;
+    typedef TS VA __attribute__((ext_vector_type(Vec16<TS>::N)));  // in LDS, aligned
     constexpr int VN = Vec16<TS>::N;
     // row strides of 16 banks (mod 32) keep the fragment reads conflict-free
     constexpr int PAD = sizeof(TS) == 8 ? 8 : 16;
@@ -222,22 +224,29 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(gemm_waves<
     const int wv = w / KSPLIT;
     const int wm = (wv % WGM) * SH::WTM, wn = (wv / WGM) * SH::WTN;
 
-    const bool full_mn = vec_ok && bm + BM <= m && bn + BN <= n;
     const int nk = (k + BK - 1) / BK;
 
     // this thread's part of a slice
     const int ar = (tid % TPA) * VN, ac = tid / TPA;  // A rows ar.., column ac + CPA * p
     const int bk = (tid % TPB) * VN, bc = tid / TPB;  // B rows bk.., column bc + CPB * p
     V ra[NPA], rb[NPB];
+    // Rows of A past m and columns of B past n only reach elements of C that are
+    // not stored, so a whole slice is fetched with 16-byte loads wherever those
+    // stay inside the operands: past a column's end they read on in memory, up to
+    // the last column's end.  16-byte loads need no more than the element's
+    // alignment (4095 x 3001 x 2047 f32, every leading dimension odd: 967 -> 420 us;
+    // element loads and slower edge tiles before).
+    const bool a_inside = bm + BM <= m;
+    const long a_last = lda >= m ? (long)(k - 1) * lda + m - VN : -1;  // the last place of a 16-byte load
 
     auto fetch = [&](int k0) {
-        if (full_mn && k0 + BK <= k) {
+        if (k0 + BK <= k && (a_inside || bm + BM - VN + (long)(k0 + BK - 1) * lda <= a_last)) {
 #pragma unroll
             for (int p = 0; p < NPA; ++p)
                 ra[p] = *(const V *)(A + (bm + ar) + (long)(k0 + ac + CPA * p) * lda);
 #pragma unroll
             for (int p = 0; p < NPB; ++p)
-                rb[p] = *(const V *)(B + (k0 + bk) + (long)(bn + bc + CPB * p) * ldb);
+                rb[p] = *(const V *)(B + (k0 + bk) + (long)min(bn + bc + CPB * p, n - 1) * ldb);
         } else {
 #pragma unroll
             for (int p = 0; p < NPA; ++p) {
@@ -265,7 +274,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(gemm_waves<
     };
     auto stage = [&](int b) {
 #pragma unroll
-        for (int p = 0; p < NPA; ++p) *(V *)&As[b][ac + CPA * p][ar] = ra[p];
+        for (int p = 0; p < NPA; ++p) *(VA *)&As[b][ac + CPA * p][ar] = ra[p];
 #pragma unroll
         for (int p = 0; p < NPB; ++p)
 #pragma unroll
@@ -353,6 +362,81 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(gemm_waves<
                     *cp = (beta == TS(0)) ? val : val + beta * *cp;
                 }
             }
+    }
+}
+
+// ---------------------------------------------------------------- small products
+// The same product where the tiles above leave most of the chip idle: what
+// bounds it then is the launch and one trip to memory, so nothing is staged.
+// A workgroup owns a 16 x 16 tile of C; its wavefronts take 16-deep chunks of k
+// in turn, read their MFMA operands straight from memory (a chunk's loads, and
+// the next chunk's, all in flight; within a chunk step u multiplies the k of
+// 4 * lk + u, so a lane's B elements lie side by side) and add their partial
+// sums in LDS in wavefront order.  f64, us: 100^3 11.2 -> 4.3, 200 x 200 x 1000
+// 37.9 -> 9.9, 64 x 64 x 4000 119 -> 37 (an empty kernel: 2.3).
+template <typename TS, int MODE>
+__global__ __launch_bounds__(512) void gemm_direct_kernel(int m, int n, int k, TS alpha, const TS *__restrict__ A,
+                                                          long lda, const TS *__restrict__ B, long ldb, TS beta,
+                                                          TS *__restrict__ C, long ldc)
+{
+    static_assert(MODE == MODE_F64 || MODE == MODE_F32, "FP64 or FP32 MFMA");
+    using AccT = typename Acc<MODE>::T;
+    constexpr int W = 8;
+    __shared__ TS part[W][4][64];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int li = lane & 15, lk = lane >> 4;
+    const int tm = (m + 15) / 16;
+    const int bm = blockIdx.x % tm * 16, bn = blockIdx.x / tm * 16;
+
+    // rows and columns past the edge only reach elements that are not stored
+    const TS *Ar = A + min(bm + li, m - 1);
+    const TS *Bc = B + (long)min(bn + li, n - 1) * ldb;
+    TS a[2][4], b[2][4];
+    auto fetch = [&](int c, TS (&x)[4], TS (&y)[4]) {
+        const int k0 = c * 16 + 4 * lk;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int g = min(k0 + u, k - 1);
+            x[u] = Ar[(long)g * lda];
+            y[u] = Bc[g];
+        }
+    };
+    AccT acc;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) acc[v] = 0;
+    auto multiply = [&](int c, const TS (&x)[4], const TS (&y)[4]) {
+        const int k0 = c * 16 + 4 * lk;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const TS xa = k0 + u < k ? x[u] : TS(0), yb = k0 + u < k ? y[u] : TS(0);
+            if constexpr (MODE == MODE_F64)
+                acc = __builtin_amdgcn_mfma_f64_16x16x4f64(yb, xa, acc, 0, 0, 0);
+            else
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(yb, xa, acc, 0, 0, 0);
+        }
+    };
+    if (k > 0) {
+        fetch(w, a[0], b[0]);
+        for (int c = w; c * 16 < k; c += 2 * W) {
+            fetch(c + W, a[1], b[1]);
+            multiply(c, a[0], b[0]);
+            fetch(c + 2 * W, a[0], b[0]);
+            multiply(c + W, a[1], b[1]);
+        }
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) part[w][v][lane] = acc[v];
+    __syncthreads();
+    if (w >= 4) return;
+    TS sum = part[0][w][lane];
+#pragma unroll
+    for (int q = 1; q < W; ++q) sum += part[q][w][lane];
+    const int row = bm + li, col = bn + (MODE == MODE_F64 ? lk + 4 * w : 4 * lk + w);
+    if (row < m && col < n) {
+        TS *cp = C + row + (long)col * ldc;
+        const TS val = alpha * sum;
+        *cp = (beta == TS(0)) ? val : val + beta * *cp;
     }
 }
 
@@ -579,17 +663,18 @@ template <typename TS, int MODE, typename SH>
 hipError_t gemm_cm_launch(hipStream_t st, int m, int n, int k, TS alpha, const TS *A, long lda, const TS *B,
                           long ldb, TS beta, TS *C, long ldc)
 {
-    constexpr int VN = Vec16<TS>::N;
-    const int vec_ok = ((uintptr_t)A % 16 == 0) && ((uintptr_t)B % 16 == 0) && lda % VN == 0 && ldb % VN == 0;
     const long tiles = (long)((m + SH::BM - 1) / SH::BM) * ((n + SH::BN - 1) / SH::BN);
     hipLaunchKernelGGL((gemm_cm_kernel<TS, MODE, SH>), dim3((unsigned)tiles), dim3(256), 0, st, m, n, k, alpha, A,
-                       lda, B, ldb, beta, C, ldc, vec_ok);
+                       lda, B, ldb, beta, C, ldc);
     return hipGetLastError();
 }
 
 // Column-major operands (or all three row-major, computed as the transposed
-// product): the largest tile shape that still gives every CU a workgroup,
-// else the split-k shape.
+// product): the largest tile shape that still gives every CU a workgroup, else
+// the split-k shape, or, where C has at most two 16 x 16 tiles per CU, no
+// staging at all (f64, us, staged and direct: 300^3, 361 tiles, 18.3 and 8.5;
+// 400^3, 625 tiles, 19.1 and 18.5; 512^3, 1024 tiles, 19.7 and 24.1; f32 at 625
+// tiles already 14.5 and 16.3).
 template <typename TS, int MODE>
 hipError_t gemm_cm(hipStream_t st, int m, int n, int k, TS alpha, const TS *A, long lda, const TS *B, long ldb,
                    TS beta, TS *C, long ldc)
@@ -600,6 +685,11 @@ hipError_t gemm_cm(hipStream_t st, int m, int n, int k, TS alpha, const TS *A, l
         return gemm_cm_launch<TS, MODE, GemmLarge>(st, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc);
     if (tiles(GemmMedium::BM) >= CUS)
         return gemm_cm_launch<TS, MODE, GemmMedium>(st, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc);
+    if (tiles(16) <= 2 * CUS) {
+        hipLaunchKernelGGL((gemm_direct_kernel<TS, MODE>), dim3((unsigned)tiles(16)), dim3(512), 0, st, m, n, k,
+                           alpha, A, lda, B, ldb, beta, C, ldc);
+        return hipGetLastError();
+    }
     return gemm_cm_launch<TS, MODE, GemmSmall>(st, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc);
 }
 

@@ -101,7 +101,9 @@ class DMatrix:
         gemm(self, alpha, a, b, beta)
 
     def __matmul__(self, other: "DMatrix") -> "DMatrix":
-        out = DMatrix.zeros(self.nrows, other.ncols, self.dtype, self.data.device)
+        # beta = 0: gemm writes every element and reads none
+        out = DMatrix(torch.empty(self.nrows * other.ncols, dtype=self.dtype, device=self.data.device), self.nrows,
+                      other.ncols)
         gemm(out, 1.0, self, other, 0.0)
         return out
 
