@@ -284,193 +284,307 @@ __global__ __launch_bounds__(64) void getrf_getrs_batched_kernel(
     }
 }
 
-// Accumulator t of dotx (src/base/blas.rs:93-167) over len products p[0..len)
-// held in LDS: positions t, t + 8, ... of the full blocks of 8, in order.  The
-// caller combines 0 + (acc0+acc4) + (acc1+acc5) + (acc2+acc6) + (acc3+acc7)
-// and adds the tail.
-__device__ __forceinline__ double dotx_acc(const double *p, int len, int t)
+// x of lane T of the eight-lane group, in lane J (T, J static)
+template <int J, int T>
+__device__ __forceinline__ double from_lane(double x)
 {
-    const int full = len & ~7;
-    double a = 0.0;
-    for (int e = t; e < full; e += 8) a += p[e];
-    return a;
+    if constexpr (J == T) {
+        return x;
+    } else {
+        constexpr int CTRL = J > T ? 0x110 + (J - T) : 0x100 + (T - J);  // row_shr, row_shl
+        const long long v = __double_as_longlong(x);
+        const int lo = __builtin_amdgcn_mov_dpp((int)v, CTRL, 0xf, 0xf, true);
+        const int hi = __builtin_amdgcn_mov_dpp((int)(v >> 32), CTRL, 0xf, 0xf, true);
+        return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+    }
 }
 
-// Adjoint of X = A^{-1} B from LU::new's packed factors and pivots, one
-// member per group of G lanes (lane r holds row r of L \ U):
+// res + x of lanes FROM, FROM + STEP, ... (COUNT of them), in that order, in lane J
+template <int J, int FROM, int STEP, int COUNT>
+__device__ __forceinline__ double add_lanes(double res, double x)
+{
+    if constexpr (COUNT > 0) {
+        res += from_lane<J, FROM>(x);
+        res = add_lanes<J, FROM + STEP, STEP, COUNT - 1>(res, x);
+    }
+    return res;
+}
+
+// The adjoint's two substitutions read a matrix column by column; a group of
+// eight lanes holds one member, lane c the solved values of index c modulo 8:
+// the eight interleaved accumulators of dotx (src/base/blas.rs:93-167) are the
+// eight lanes.  The columns are fetched AHEAD steps before their use.
+constexpr int AHEAD = 4;
+
+template <int KM>
+struct Column {
+    double x[KM];  // the elements that meet solved blocks 0, 1, ...
+    double cur;    // those of the block in work
+};
+
+// ---- U^T y = g, i = 8 kb + J ascending: the products of whole blocks of 8
+// before i in the lanes' accumulators, those of i's own block one after another.
+template <int KM, int CH, int J>
+__device__ __forceinline__ void upper_step(int kb, int c, const Column<KM> &u, const double (&z)[CH][KM],
+                                           double (&cur)[CH], const double (&gv)[CH])
+{
+#pragma unroll
+    for (int q = 0; q < CH; ++q) {
+        double acc = 0.0;
+#pragma unroll
+        for (int k = 0; k < KM; ++k) {
+            const double p = u.x[k] * z[q][k];
+            acc += k < kb ? p : 0.0;
+        }
+        const double tail = u.cur * cur[q];
+        const double pair = acc + from_lane<0, 4>(acc);  // in lanes 0..3
+        double res = add_lanes<J, 0, 1, 4>(0.0, pair);
+        res = add_lanes<J, 0, 1, J>(res, tail);
+        const double y = (gv[q] - res) / u.cur;  // in lane J
+        cur[q] = c == J ? y : cur[q];
+    }
+}
+
+// accumulators 0..3 (each with its pair) of step J of the descending pass: T = 0..3
+template <int J, int T>
+__device__ __forceinline__ double add_pairs(double res, double pair)
+{
+    if constexpr (T < 4) {
+        res += from_lane<J, (J + 7 - T) & 3>(pair);
+        res = add_pairs<J, T + 1>(res, pair);
+    }
+    return res;
+}
+
+// ---- L^T z = y, i = n - 1 - s descending, s = 8 kb + J: counted from the end
+// (e = n - 1 - row), the dot runs over e = s - 1 down to 0, so its whole blocks
+// of 8 end at e = J and the tail is e = J - 1 .. 0.  Accumulator t holds the e
+// with e = J - 1 - t modulo 8.
+template <int KM, int CH, int J>
+__device__ __forceinline__ void lower_step(int kb, int c, const Column<KM> &l, const double (&z)[CH][KM],
+                                           double (&cur)[CH], const double (&yv)[CH])
+{
+#pragma unroll
+    for (int q = 0; q < CH; ++q) {
+        const double pc = l.cur * cur[q];
+        double acc = 0.0;
+        acc += (kb > 0 && c < J) ? pc : 0.0;
+        double p0 = 0.0;
+#pragma unroll
+        for (int k = KM - 1; k >= 0; --k) {
+            const double p = l.x[k] * z[q][k];
+            acc += (k < kb && (k > 0 || c >= J)) ? p : 0.0;
+            if (k == 0) p0 = p;
+        }
+        const double tail = kb > 0 ? p0 : pc;
+        const double pair = acc + from_lane<0, 4>(acc);  // in lanes 0..3
+        double res = add_pairs<J, 0>(0.0, pair);
+        res = add_lanes<J, J - 1, -1, J>(res, tail);
+        cur[q] = c == J ? yv[q] - res : cur[q];  // the unit diagonal divides by one
+    }
+}
+
+template <int KM>
+__device__ __forceinline__ void fetch_upper(Column<KM> &u, const double *M, int n, int i, int c)
+{
+    i = min(i, n - 1);
+    const double *col = M + (size_t)i * n;
+#pragma unroll
+    for (int k = 0; k < KM; ++k) u.x[k] = col[min(8 * k + c, i)];
+    u.cur = col[min((i & ~7) + c, i)];
+}
+
+template <int KM>
+__device__ __forceinline__ void fetch_lower(Column<KM> &l, const double *M, int n, int s, int c)
+{
+    s = min(s, n - 1);
+    const int i = n - 1 - s, top = min(i + 1, n - 1);
+    const double *col = M + (size_t)i * n;
+#pragma unroll
+    for (int k = 0; k < KM; ++k) l.x[k] = col[max(n - 1 - 8 * k - c, top)];
+    l.cur = col[max(n - 1 - (s & ~7) - c, top)];
+}
+
+template <int KM, int CH, bool UPPER, int J>
+__device__ __forceinline__ void block_steps(int kb, int c, Column<KM> (&ring)[AHEAD], const double *M, int n,
+                                            const double (&z)[CH][KM], double (&cur)[CH], const double (&gv)[CH])
+{
+    if constexpr (J < 8) {
+        if constexpr (UPPER) {
+            upper_step<KM, CH, J>(kb, c, ring[J % AHEAD], z, cur, gv);
+            fetch_upper<KM>(ring[J % AHEAD], M, n, 8 * kb + J + AHEAD, c);
+        } else {
+            lower_step<KM, CH, J>(kb, c, ring[J % AHEAD], z, cur, gv);
+            fetch_lower<KM>(ring[J % AHEAD], M, n, 8 * kb + J + AHEAD, c);
+        }
+        block_steps<KM, CH, UPPER, J + 1>(kb, c, ring, M, n, z, cur, gv);
+    }
+}
+
+// One substitution over v (the group's values by row, overwritten by the result).
+template <int KM, int CH, int LD, bool UPPER>
+__device__ __forceinline__ void substitute(const double *M, int n, int blocks, int c, double (*v)[LD])
+{
+    Column<KM> ring[AHEAD];
+#pragma unroll
+    for (int s = 0; s < AHEAD; ++s) {
+        if constexpr (UPPER) fetch_upper<KM>(ring[s], M, n, s, c);
+        else fetch_lower<KM>(ring[s], M, n, s, c);
+    }
+    double z[CH][KM];
+#pragma unroll
+    for (int q = 0; q < CH; ++q)
+#pragma unroll
+        for (int k = 0; k < KM; ++k) z[q][k] = 0.0;
+    for (int kb = 0; kb < blocks; ++kb) {
+        const int e = 8 * kb + c, row = UPPER ? e : n - 1 - e;
+        double gv[CH], cur[CH];
+#pragma unroll
+        for (int q = 0; q < CH; ++q) {
+            gv[q] = v[q][max(row, 0)];
+            cur[q] = 0.0;
+        }
+        block_steps<KM, CH, UPPER, 0>(kb, c, ring, M, n, z, cur, gv);
+#pragma unroll
+        for (int q = 0; q < CH; ++q) {
+#pragma unroll
+            for (int k = 0; k < KM; ++k) z[q][k] = k == kb ? cur[q] : z[q][k];
+            if (e < n) v[q][row] = cur[q];
+        }
+    }
+}
+
+// Adjoint of X = A^{-1} B from LU::new's packed factors and pivots:
 //   U^T y = g  (tr_solve_upper_triangular, solve.rs:255-276,411-440),
 //   L^T z = y  (tr_solve_lower_triangular on the unit L, solve.rs:232-253,379-409),
 //   Lambda = P^T z (inv_permute_rows, permutation_sequence.rs:108-116),
 //   dB = Lambda, dA = -Lambda X^T (products summed over right-hand sides in
 //   order), each dot in dotx's order.
-template <int NB, int G>
-__global__ __launch_bounds__(64) void getrs_backward_batched_kernel(
-    const int *__restrict__ order, int begin, int end, const int *__restrict__ nsz,
-    const double *const *__restrict__ LUptr, const int *const *__restrict__ Pptr,
-    const double *const *__restrict__ Xptr, const double *const *__restrict__ dXptr,
-    double *const *__restrict__ dAptr, double *const *__restrict__ dBptr, int nrhs)
+//
+// Bound by the chain of dots, one per row: products, up to 8 additions, the
+// joining of the accumulators and the tail, about 300 cycles a step.  One
+// member's chain uses few lanes, so eight members share a wavefront (eight lanes
+// each, the accumulators of a dot side by side), nothing of a step crosses a
+// group, and no step needs a barrier; members of the whole range of sizes run in
+// one launch, the largest first.  Before, a member had 16 to 64 lanes, a dot
+// three barriers and each range of sizes its own launch: 16384 members of
+// n = 4..64, 2 right-hand sides, 2250 -> 177 us, where reading the factors and
+// writing dA take 85.
+// KM: blocks of 8 rows that a lane can hold; CH: right-hand sides at a time.
+template <int KM, int CH>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void getrs_backward_batched_kernel(
+    const int *__restrict__ order, int count, const int *__restrict__ nsz, const double *const *__restrict__ LUptr,
+    const int *const *__restrict__ Pptr, const double *const *__restrict__ Xptr,
+    const double *const *__restrict__ dXptr, double *const *__restrict__ dAptr, double *const *__restrict__ dBptr,
+    int nrhs)
 {
-    constexpr int MPW = 64 / G;
-    __shared__ double prod[MPW][CH][NB];
-    __shared__ double accs[MPW][CH][8];
-    __shared__ double vbuf[MPW][CH][NB];  // z then Lambda, by position; X rows for dA
+    constexpr int NB = 8 * KM, LD = NB + 1;
+    __shared__ double v[8][CH][LD];   // a chunk's values by row: g, y, z, Lambda
+    __shared__ double xs[8][CH][LD];  // the chunk of X
+    __shared__ int swap[8][NB];
     const int lane = threadIdx.x;
-    const int g = lane / G, r = lane % G;
-    const int item = begin + (int)blockIdx.x * MPW + g;
-    const bool valid = item < end;
+    const int g = lane >> 3, c = lane & 7;
+    const int item = (int)blockIdx.x * 8 + g;
+    const bool valid = item < count;
     const int jm = valid ? order[item] : 0;
     const int n = valid ? nsz[jm] : 0;
-    const double *const LU = valid ? LUptr[jm] : nullptr;
-    const int *const P = valid ? Pptr[jm] : nullptr;
-    const double *const X = valid ? Xptr[jm] : nullptr;
-    const double *const dX = valid ? dXptr[jm] : nullptr;
-    double *const dA = valid ? dAptr[jm] : nullptr;
-    double *const dB = valid ? dBptr[jm] : nullptr;
-    const bool row_ok = r < n;
-
-    double a[NB];
-    {
-        const double *row = row_ok ? LU + r : kZeroCellLU;
-        const size_t step = row_ok ? (size_t)n : 0;
+    int most = n;
 #pragma unroll
-        for (int c = 0; c < NB; ++c) {
-            const double *src = (c < n) ? row + (size_t)c * step : kZeroCellLU;
-            a[c] = *src;
-        }
+    for (int off = 8; off < 64; off *= 2) most = max(most, __shfl_xor(most, off));
+    const int blocks = __builtin_amdgcn_readfirstlane((most + 7) >> 3);
+    if (blocks == 0) return;
+    // a group without a member, or with an empty one, walks a 1 x 1 zero
+    const double *const LU = n > 0 ? LUptr[jm] : kZeroCellLU;
+    const int nm = max(n, 1);
+    if (n > 0) {
+        const int *const P = Pptr[jm];
+        for (int i = c; i < n; i += 8) swap[g][i] = P[i];
     }
     for (int c0 = 0; c0 < nrhs; c0 += CH) {
-        const int qn = nrhs - c0 < CH ? nrhs - c0 : CH;
-        double y[CH];
+        const double *const dX = n > 0 ? dXptr[jm] : nullptr;
+        for (int i = c; i < n; i += 8)
 #pragma unroll
-        for (int q = 0; q < CH; ++q) y[q] = (row_ok && q < qn) ? dX[r + (size_t)(c0 + q) * n] : 0.0;
-        // ---- U^T y = g, i ascending: y_i = (g_i - dotx(U[0..i, i], y[0..i])) / U_ii
-#pragma unroll
-        for (int i = 0; i < NB; ++i) {
-            const bool live = i < n;
-            if (r < NB) {
-#pragma unroll
-                for (int q = 0; q < CH; ++q) prod[g][q][r] = a[i] * y[q];
-            }
-            __syncthreads();
-            if (live && r < 8) {
-#pragma unroll
-                for (int q = 0; q < CH; ++q) accs[g][q][r] = dotx_acc(prod[g][q], i, r);
-            }
-            __syncthreads();
-            if (live && r == i) {
-                const int full = i & ~7;
-#pragma unroll
-                for (int q = 0; q < CH; ++q) {
-                    const double *ac = accs[g][q];
-                    double res = 0.0;
-                    res += ac[0] + ac[4];
-                    res += ac[1] + ac[5];
-                    res += ac[2] + ac[6];
-                    res += ac[3] + ac[7];
-                    for (int e = full; e < i; ++e) res += prod[g][q][e];
-                    y[q] = (y[q] - res) / a[i];
-                }
-            }
-            __syncthreads();
-        }
-        // ---- L^T z = y, i descending: z_i = (y_i - dotx(L[i+1.., i], z[i+1..])) / 1
-#pragma unroll
-        for (int i = NB - 1; i >= 0; --i) {
-            const bool live = i < n;
-            if (r < NB) {
-#pragma unroll
-                for (int q = 0; q < CH; ++q) prod[g][q][r] = a[i] * y[q];
-            }
-            __syncthreads();
-            const int len = n - i - 1;
-            if (live && r < 8) {
-#pragma unroll
-                for (int q = 0; q < CH; ++q) accs[g][q][r] = len > 0 ? dotx_acc(prod[g][q] + i + 1, len, r) : 0.0;
-            }
-            __syncthreads();
-            if (live && r == i) {
-                const int full = len > 0 ? (len & ~7) : 0;
-#pragma unroll
-                for (int q = 0; q < CH; ++q) {
-                    const double *ac = accs[g][q];
-                    double res = 0.0;
-                    res += ac[0] + ac[4];
-                    res += ac[1] + ac[5];
-                    res += ac[2] + ac[6];
-                    res += ac[3] + ac[7];
-                    for (int e = full; e < len; ++e) res += prod[g][q][i + 1 + e];
-                    y[q] = (y[q] - res) / 1.0;
-                }
-            }
-            __syncthreads();
-        }
-        // ---- Lambda = P^T z: the swaps (i, ipiv[i]) in reverse order
-        if (row_ok) {
-#pragma unroll
-            for (int q = 0; q < CH; ++q) vbuf[g][q][r] = y[q];
-        }
+            for (int q = 0; q < CH; ++q) v[g][q][i] = c0 + q < nrhs ? dX[i + (size_t)(c0 + q) * n] : 0.0;
         __syncthreads();
-        if (valid && r == 0) {
+        substitute<KM, CH, LD, true>(LU, nm, blocks, c, v[g]);
+        __syncthreads();
+        substitute<KM, CH, LD, false>(LU, nm, blocks, c, v[g]);
+        __syncthreads();
+        // the swaps (i, ipiv[i]) in reverse order, a lane per right-hand side
+        if (c < CH) {
+            double *const col = v[g][c];
             for (int i = n - 1; i >= 0; --i) {
-                const int pv = P[i];
-                if (pv != i) {
-#pragma unroll
-                    for (int q = 0; q < CH; ++q) {
-                        const double t = vbuf[g][q][i];
-                        vbuf[g][q][i] = vbuf[g][q][pv];
-                        vbuf[g][q][pv] = t;
-                    }
-                }
+                const int pv = swap[g][i];
+                const double t = col[i], o = col[pv];
+                col[i] = o;
+                col[pv] = t;
             }
         }
         __syncthreads();
-        double lam[CH];
-#pragma unroll
-        for (int q = 0; q < CH; ++q) lam[q] = row_ok ? vbuf[g][q][r] : 0.0;
-        if (row_ok) {
+        double *const dB = n > 0 ? dBptr[jm] : nullptr;
+        for (int i = c; i < n; i += 8)
 #pragma unroll
             for (int q = 0; q < CH; ++q)
-                if (q < qn) dB[r + (size_t)(c0 + q) * n] = lam[q];
-        }
+                if (c0 + q < nrhs) dB[i + (size_t)(c0 + q) * n] = v[g][q][i];
         __syncthreads();
-        // ---- dA[r, c] = -(sum over right-hand sides of fl(Lambda_r * X_c)), X rows through LDS
-        if (row_ok) {
+    }
+    // dA[r, k] = -(sum over right-hand sides of fl(Lambda_r * X_k)), the whole
+    // wavefront on one member at a time, along its columns
+    for (int c0 = 0; c0 == 0 || c0 < nrhs; c0 += CH) {
+        const int qn = min(nrhs - c0, CH);
+        const double *const X = n > 0 && qn > 0 ? Xptr[jm] : nullptr;
+        const double *const dB = n > 0 && qn > 0 ? dBptr[jm] : nullptr;
+        for (int i = c; i < n; i += 8)
 #pragma unroll
-            for (int q = 0; q < CH; ++q) vbuf[g][q][r] = (q < qn) ? X[r + (size_t)(c0 + q) * n] : 0.0;
-        }
+            for (int q = 0; q < CH; ++q) {
+                if (q >= qn) break;
+                xs[g][q][i] = X[i + (size_t)(c0 + q) * n];
+                if (nrhs > CH) v[g][q][i] = dB[i + (size_t)(c0 + q) * n];
+            }
         __syncthreads();
-        if (row_ok) {
-            for (int c = 0; c < n; ++c) {
-                double sacc = c0 > 0 ? -dA[r + (size_t)c * n] : 0.0;
+        const unsigned long long dA = n > 0 ? (unsigned long long)dAptr[jm] : 0;
+        for (int m = 0; m < 8; ++m) {
+            const int mn = __builtin_amdgcn_readlane(n, 8 * m);
+            if (mn == 0) continue;
+            double *const D = (double *)((unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)dA, 8 * m) |
+                                         (unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(dA >> 32), 8 * m) << 32);
+            const int dk = 64 / mn, dr = 64 - dk * mn;
+            int k = lane / mn, r = lane - k * mn;
+            for (int e = lane; e < mn * mn; e += 64) {
+                double s = c0 > 0 ? -D[e] : 0.0;
 #pragma unroll
                 for (int q = 0; q < CH; ++q) {
                     if (q < qn) {
-                        const double pr = lam[q] * vbuf[g][q][c];
-                        sacc = (c0 == 0 && q == 0) ? pr : sacc + pr;
+                        const double pr = v[m][q][r] * xs[m][q][k];
+                        s = (c0 == 0 && q == 0) ? pr : s + pr;
                     }
                 }
-                dA[r + (size_t)c * n] = -sacc;
+                D[e] = qn > 0 ? -s : 0.0;  // no right-hand sides: zero
+                r += dr;
+                k += dk;
+                if (r >= mn) {
+                    r -= mn;
+                    ++k;
+                }
             }
         }
         __syncthreads();
     }
-    // no right-hand sides: X and its gradient are empty
-    if (nrhs == 0 && row_ok)
-        for (int c = 0; c < n; ++c) dA[r + (size_t)c * n] = 0.0;
 }
 
-template <int NB>
-int launch_bwd_nb(hipStream_t st, const int *order, int begin, int end, const int *nsz, const double *const *LU,
-                  const int *const *P, const double *const *X, const double *const *dX, double *const *dA,
-                  double *const *dB, int nrhs)
+// One launch for the whole batch: `order` holds the members by decreasing size.
+template <int KM>
+void launch_bwd(hipStream_t st, const int *order, int count, const int *nsz, const double *const *LU,
+                const int *const *P, const double *const *X, const double *const *dX, double *const *dA,
+                double *const *dB, int nrhs)
 {
-    constexpr int G = group_for<NB>();
-    constexpr int MPW = 64 / G;
-    const unsigned grid = (unsigned)((end - begin + MPW - 1) / MPW);
-    if (grid == 0) return 0;
-    hipLaunchKernelGGL((getrs_backward_batched_kernel<NB, G>), dim3(grid), dim3(64), 0, st, order, begin, end, nsz,
-                       LU, P, X, dX, dA, dB, nrhs);
-    return hipGetLastError() == hipSuccess ? 0 : 1;
+    const dim3 grid((unsigned)((count + 7) / 8));
+    if (nrhs > 1)
+        hipLaunchKernelGGL((getrs_backward_batched_kernel<KM, 2>), grid, dim3(64), 0, st, order, count, nsz, LU, P, X,
+                           dX, dA, dB, nrhs);
+    else
+        hipLaunchKernelGGL((getrs_backward_batched_kernel<KM, 1>), grid, dim3(64), 0, st, order, count, nsz, LU, P, X,
+                           dX, dA, dB, nrhs);
 }
 
 template <int NB>
@@ -494,10 +608,6 @@ using Launch = int (*)(bool, hipStream_t, const int *, int, int, const int *, do
                        double *const *, int, int *);
 const Launch kLaunch[8] = {launch_nb<8>, launch_nb<16>, launch_nb<24>, launch_nb<32>,
                            launch_nb<40>, launch_nb<48>, launch_nb<56>, launch_nb<64>};
-using BwdLaunch = int (*)(hipStream_t, const int *, int, int, const int *, const double *const *, const int *const *,
-                          const double *const *, const double *const *, double *const *, double *const *, int);
-const BwdLaunch kBwdLaunch[8] = {launch_bwd_nb<8>,  launch_bwd_nb<16>, launch_bwd_nb<24>, launch_bwd_nb<32>,
-                                 launch_bwd_nb<40>, launch_bwd_nb<48>, launch_bwd_nb<56>, launch_bwd_nb<64>};
 
 }  // namespace
 
@@ -542,11 +652,11 @@ extern "C" int nrocm_dgetrs_backward_batched(nrocm_handle h, nrocm_batch bt, con
     if (bt->count > 0 && bt->nrhs > 0 && !db) return -8;
     if (bt->count == 0) return NROCM_OK;
     if (bt->max_n > 64) return nrocm_fail(h, NROCM_ERR_UNSUPPORTED, "batched LU adjoint supports n <= 64");
-    for (const auto &bin : bt->bins) {
-        if (bin.end <= bin.begin) continue;
-        if (kBwdLaunch[bin.kernel](h->stream, bt->order_dev, bin.begin, bin.end, bt->n_dev, lu, ipiv, x, dx, da, db,
-                                   bt->nrhs))
-            NROCM_CHECK_LAUNCH(h);
-    }
+    // up to 32 rows a lane holds half as many values, and the dots have half the terms
+    if (bt->max_n <= 32)
+        launch_bwd<4>(h->stream, bt->order_dev, bt->count, bt->n_dev, lu, ipiv, x, dx, da, db, bt->nrhs);
+    else
+        launch_bwd<8>(h->stream, bt->order_dev, bt->count, bt->n_dev, lu, ipiv, x, dx, da, db, bt->nrhs);
+    NROCM_CHECK_LAUNCH(h);
     return NROCM_OK;
 }
