@@ -416,7 +416,7 @@ hipError_t window_panel(hipStream_t st, T *A, int lda, int n, int k0, int *ipiv,
 {
     const int nb = std::min(64, n - k0);
     const int kw = std::min(n, k0 + WINDOW_ROWS);
-    hipLaunchKernelGGL((window_panel_kernel<T>), dim3(1), dim3(WINDOW_ROWS), 0, st, A, lda, k0, nb, kw, ipiv, info,
+    hipLaunchKernelGGL((window_panel_kernel<T>), dim3(1), dim3(512), 0, st, A, lda, k0, nb, kw, ipiv, info,
                        plan, perm);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || kw >= n) return e;
