@@ -250,10 +250,10 @@ int nrocm_dqr_rsolve(nrocm_handle handle, int n, const double *qr, int lda,
                      const double *diag, int nrhs, double *b, int ldb, int *info);
 
 /* Batched tall least squares, min ||A_j x - b_j||, A_j m_j x n (f32, lda m_j,
- * n <= m_j <= 2048, n <= 64), batch created with the row counts m_j.  Blocked
- * compact-WY Householder QR of a workspace copy of [A_j | b_j] (LAPACK
- * sgeqrf/slarft conventions) with the WY products V^T C and C - V (T^T W) on
- * FP32 MFMA, x = R^{-1} (Q^T b)[0..n), then `refine` FP64 residual-refinement
+ * n <= m_j <= 2048, n <= 64), batch created with the row counts m_j.  Householder
+ * QR in blocks of 128 rows, each reduced into R (LAPACK's reflector conventions;
+ * compact-WY products on FP32 MFMA), Q^T b in FP64 from the FP32 reflectors,
+ * x = R^{-1} (Q^T b)[0..n), then `refine` FP64 residual-refinement
  * steps x += R^{-1} (Q^T (b - A x))[0..n) with b - A x formed in FP64.  A_j and
  * b_j are not modified; x is n x count f64 (column j = system j); info[j] = 0 or
  * 1 + index of a zero R diagonal.  Replaces the tall solve nalgebra-lapack's

@@ -333,14 +333,21 @@ int nrocm_batch_create(nrocm_handle h, int count, const int *n_host, int nrhs, n
         pos = endp;
     }
     if (count > 0) {
-        if (hipMalloc(&bt->order_dev, sizeof(int) * count) != hipSuccess ||
-            hipMalloc(&bt->n_dev, sizeof(int) * count) != hipSuccess) {
+        std::vector<int> blocks(count);
+        for (int j = 0; j < count; ++j) {
+            blocks[j] = (int)bt->row_blocks;
+            bt->row_blocks += (n_host[j] + 127LL) / 128;
+        }
+        if (hipMalloc(&bt->order_dev, sizeof(int) * 3 * (size_t)count) != hipSuccess) {
             nrocm_batch_destroy(bt);
             return NROCM_ERR_ALLOC;
         }
+        bt->n_dev = bt->order_dev + count;
+        bt->blocks_dev = bt->n_dev + count;
         if (hipMemcpy(bt->order_dev, bt->order_host.data(), sizeof(int) * count,
                       hipMemcpyHostToDevice) != hipSuccess ||
-            hipMemcpy(bt->n_dev, n_host, sizeof(int) * count, hipMemcpyHostToDevice) != hipSuccess) {
+            hipMemcpy(bt->n_dev, n_host, sizeof(int) * count, hipMemcpyHostToDevice) != hipSuccess ||
+            hipMemcpy(bt->blocks_dev, blocks.data(), sizeof(int) * count, hipMemcpyHostToDevice) != hipSuccess) {
             nrocm_batch_destroy(bt);
             return NROCM_ERR_HIP;
         }
@@ -355,7 +362,6 @@ int nrocm_batch_destroy(nrocm_batch bt)
     drop_graphs(bt);
     if (bt->graph_stream) (void)hipStreamDestroy(bt->graph_stream);
     if (bt->order_dev) (void)hipFree(bt->order_dev);
-    if (bt->n_dev) (void)hipFree(bt->n_dev);
     delete bt;
     return NROCM_OK;
 }

@@ -13,6 +13,7 @@
 #include "solve_sweep.hpp"
 
 #include <algorithm>
+#include <utility>
 #include <cmath>
 
 namespace {
