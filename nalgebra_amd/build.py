@@ -24,7 +24,7 @@ ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 HIPCC = os.path.join(ROCM, "bin", "hipcc")
 ARCH = "gfx950"
 
-HIP_SOURCES = ["chol_batched.hip", *[f"chol_nb{nb:02d}.hip" for nb in range(8, 65, 8)],
+HIP_SOURCES = ["chol_batched.hip", "chol_adjoint.hip", *[f"chol_nb{nb:02d}.hip" for nb in range(8, 65, 8)],
                "lu.hip", "gemm.hip", "qr.hip", "mixed.hip", "solve_small.hip", "solve_lookback.hip", "lu_batched.hip"]
 HOST_SOURCES = ["runtime.cpp"]
 

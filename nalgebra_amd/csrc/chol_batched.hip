@@ -30,9 +30,6 @@ using FacLaunch = int (*)(bool, unsigned, hipStream_t, const int *, int, int, co
 using SolLaunch = int (*)(bool, unsigned, hipStream_t, const int *, int, int, const int *,
                          double *const *, double *const *, int, const int *, double *, double *,
                          int, int, int);
-using BwdLaunch = int (*)(unsigned, hipStream_t, const int *, int, int, const int *,
-                         const double *const *, const double *const *, const double *const *,
-                         double *const *, double *const *, int);
 using FusedLaunch = int (*)(bool, int, hipStream_t, const int *, int, int, const int *, double *const *,
                            double *const *, int, int *);
 
@@ -44,10 +41,6 @@ const SolLaunch kSol[8] = {nrocm_chol_potrs_launch_8,  nrocm_chol_potrs_launch_1
                            nrocm_chol_potrs_launch_24, nrocm_chol_potrs_launch_32,
                            nrocm_chol_potrs_launch_40, nrocm_chol_potrs_launch_48,
                            nrocm_chol_potrs_launch_56, nrocm_chol_potrs_launch_64};
-const BwdLaunch kBwd[8] = {nrocm_chol_bwd_launch_8,  nrocm_chol_bwd_launch_16,
-                           nrocm_chol_bwd_launch_24, nrocm_chol_bwd_launch_32,
-                           nrocm_chol_bwd_launch_40, nrocm_chol_bwd_launch_48,
-                           nrocm_chol_bwd_launch_56, nrocm_chol_bwd_launch_64};
 
 const FusedLaunch kFused[8] = {nrocm_chol_fused_launch_8,  nrocm_chol_fused_launch_16,
                                nrocm_chol_fused_launch_24, nrocm_chol_fused_launch_32,
@@ -91,8 +84,6 @@ int default_lanes(int bin)
     const int nb = 8 * (bin + 1);
     return nb <= 8 ? 8 : nb <= 16 ? 16 : nb <= 32 ? 32 : 64;
 }
-
-int mpw_of_bin(int bin) { return 64 / default_lanes(bin); }
 
 // The bins are independent.  With `split`, the bins (sizes in decreasing
 // order) are dealt round-robin to the stream and kBranches - 1 auxiliary
@@ -466,31 +457,6 @@ int nrocm_dpotrf_potrs_batched(nrocm_handle h, nrocm_batch bt, double *const *A,
         hit = &bt->graphs.back();
     }
     NROCM_CHECK_HIP(h, hipGraphLaunch(hit->exec, h->stream));
-    return NROCM_OK;
-}
-
-int nrocm_dpotrs_backward_batched(nrocm_handle h, nrocm_batch bt, const double *const *L,
-                                  const double *const *X, const double *const *dX,
-                                  double *const *dA, double *const *dB)
-{
-    if (!h) return -1;
-    if (!bt || bt->handle != h) return -2;
-    if (bt->count > 0 && (!L)) return -3;
-    if (bt->count > 0 && (!X)) return -4;
-    if (bt->count > 0 && (!dX)) return -5;
-    if (bt->count > 0 && (!dA)) return -6;
-    if (bt->count > 0 && (!dB)) return -7;
-    if (bt->count == 0) return NROCM_OK;
-    if (bt->max_n > 64)
-        return nrocm_fail(h, NROCM_ERR_UNSUPPORTED, "batched Cholesky adjoint supports n <= 64");
-    for (const auto &bin : bt->bins) {
-        const int items = bin.end - bin.begin;
-        if (items <= 0) continue;
-        const int mpw = mpw_of_bin(bin.kernel);
-        if (kBwd[bin.kernel](nrocm_cdiv(items, mpw), h->stream, bt->order_dev, bin.begin, bin.end,
-                             bt->n_dev, L, X, dX, dA, dB, bt->nrhs))
-            NROCM_CHECK_LAUNCH(h);
-    }
     return NROCM_OK;
 }
 

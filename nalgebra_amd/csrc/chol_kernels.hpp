@@ -155,11 +155,6 @@ __device__ __forceinline__ int factor(double (&a)[NB], double *col, double *xch,
     return m ? (int)__builtin_ctzll(m) + 1 : 0;
 }
 
-__device__ __forceinline__ double reg_q(const double (&b)[CH], int q)
-{
-    return q == 0 ? b[0] : q == 1 ? b[1] : q == 2 ? b[2] : b[3];
-}
-
 constexpr int PF = 8;  // substitution steps whose L elements are loaded ahead
 
 // Forward substitution L y = b (solve.rs:488-519) for CH right-hand sides:
@@ -685,79 +680,6 @@ void potrf_potrs_kernel(const int *__restrict__ order, int begin, int end,
     }
 }
 
-// Adjoint of X = A^{-1} B given L: Lambda = (L L^T)^{-1} dX (same arithmetic as
-// Cholesky::solve_mut), dB = Lambda, dA = -1/2 (Lambda X^T + X Lambda^T).
-template <int NB, int G, bool EXACT>
-__global__ __launch_bounds__(64) void potrs_backward_kernel(
-    const int *__restrict__ order, int begin, int end, const int *__restrict__ nsz,
-    const double *const *__restrict__ Lptr, const double *const *__restrict__ Xptr,
-    const double *const *__restrict__ dXptr, double *const *__restrict__ dAptr,
-    double *const *__restrict__ dBptr, int nrhs)
-{
-    constexpr int MPW = 64 / G;
-    __shared__ Smem<MPW> s;
-    __shared__ double lam_s[2][64 * CH];
-    const int lane = threadIdx.x;
-    const int g = lane / G, r = lane % G;
-    const int item = begin + (int)blockIdx.x * MPW + g;
-    const bool valid = item < end;
-    int jm = valid ? order[item] : 0;
-    const int n = valid ? nsz[jm] : 0;
-    const double *L = valid ? Lptr[jm] : nullptr;
-    const double *X = valid ? Xptr[jm] : nullptr;
-    const double *dX = valid ? dXptr[jm] : nullptr;
-    double *dA = valid ? dAptr[jm] : nullptr;
-    double *dB = valid ? dBptr[jm] : nullptr;
-    const int nmax = __builtin_amdgcn_readfirstlane(n);
-
-    // the diagonal of L, published for the substitutions; padding rows get 1
-    s.diag[lane] = (r < n) ? L[r + (size_t)r * n] : 1.0;
-    lds_barrier();
-
-    for (int c0 = 0; c0 < nrhs; c0 += CH) {
-        double b[CH], x[CH];
-#pragma unroll
-        for (int q = 0; q < CH; ++q) {
-            const bool in = r < n && c0 + q < nrhs;
-            b[q] = in ? dX[r + (size_t)(c0 + q) * n] : 0.0;
-            x[q] = in ? X[r + (size_t)(c0 + q) * n] : 0.0;
-        }
-        forward<G, EXACT>(L, n, b, s, n, nmax, g, r, lane);
-        backward<G, EXACT>(L, n, b, s, n, nmax, g, r, lane);
-        if (r < n) {
-#pragma unroll
-            for (int q = 0; q < CH; ++q)
-                if (c0 + q < nrhs) dB[r + (size_t)(c0 + q) * n] = b[q];
-        }
-        // dA[r, c] = -1/2 (lam_r x_c + x_r lam_c), summed over right-hand sides in order
-#pragma unroll
-        for (int q = 0; q < CH; ++q) {
-            lam_s[0][lane * CH + q] = b[q];
-            lam_s[1][lane * CH + q] = x[q];
-        }
-        lds_barrier();
-        const int nq = nrhs - c0 < CH ? nrhs - c0 : CH;
-        if (r < n) {
-            for (int c = 0; c < n; ++c) {
-                double v = c0 > 0 ? dA[r + (size_t)c * n] : 0.0;
-                for (int q = 0; q < nq; ++q) {
-                    const double lc = lam_s[0][(g * G + c) * CH + q];
-                    const double xc = lam_s[1][(g * G + c) * CH + q];
-                    const double p = reg_q(b, q) * xc;
-                    const double t = reg_q(x, q) * lc;
-                    const double d = -0.5 * (p + t);
-                    v = (c0 == 0 && q == 0) ? d : v + d;
-                }
-                dA[r + (size_t)c * n] = v;
-            }
-        }
-        lds_barrier();
-    }
-    // no right-hand sides: X = A^{-1} B is empty and so is its gradient
-    if (nrhs == 0 && r < n)
-        for (int c = 0; c < n; ++c) dA[r + (size_t)c * n] = 0.0;
-}
-
 // Launches the fused kernel for members [begin, end) of `order` with G lanes
 // per matrix (64 / G matrices per wavefront).
 template <int NB, int G>
@@ -801,10 +723,6 @@ int fused_dispatch(bool exact, int G, hipStream_t st, const int *order, int begi
                                      int begin, int end, const int *nsz, double *const *A,        \
                                      double *const *B, int nrhs, const int *info, double *A1,     \
                                      double *B1, int n1, int lda1, int ldb1);                     \
-    int nrocm_chol_bwd_launch_##NB(unsigned grid, hipStream_t st, const int *order, int begin,    \
-                                   int end, const int *nsz, const double *const *L,               \
-                                   const double *const *X, const double *const *dX,               \
-                                   double *const *dA, double *const *dB, int nrhs);               \
     int nrocm_chol_fused_launch_##NB(bool exact, int G, hipStream_t st, const int *order,         \
                                      int begin, int end, const int *nsz, double *const *A,        \
                                      double *const *B, int nrhs, int *info);
@@ -837,17 +755,6 @@ int fused_dispatch(bool exact, int G, hipStream_t st, const int *order, int begi
         else                                                                                      \
             hipLaunchKernelGGL((potrs_kernel<NB, G, false>), dim3(grid), dim3(64), 0, st, order,  \
                                begin, end, nsz, A, B, nrhs, info, A1, B1, n1, lda1, ldb1);        \
-        return hipGetLastError() == hipSuccess ? 0 : 1;                                           \
-    }                                                                                             \
-    int nrocm_chol_bwd_launch_##NB(unsigned grid, hipStream_t st, const int *order, int begin,    \
-                                   int end, const int *nsz, const double *const *L,               \
-                                   const double *const *X, const double *const *dX,               \
-                                   double *const *dA, double *const *dB, int nrhs)                \
-    {                                                                                             \
-        using namespace nrocm_chol;                                                               \
-        constexpr int G = group_for<NB>();                                                        \
-        hipLaunchKernelGGL((potrs_backward_kernel<NB, G, true>), dim3(grid), dim3(64), 0, st,     \
-                           order, begin, end, nsz, L, X, dX, dA, dB, nrhs);                       \
         return hipGetLastError() == hipSuccess ? 0 : 1;                                           \
     }                                                                                             \
     int nrocm_chol_fused_launch_##NB(bool exact, int G, hipStream_t st, const int *order,         \

@@ -22,9 +22,12 @@
 // lower factor (solve.rs:106-133) and backward substitution with U
 // (solve.rs:137-182) broadcast the solved value of position i from the lane
 // holding that position, and x is stored at the row's final position.
+#include "adjoint_steps.hpp"
 #include "internal_launch.hpp"
 
 #include <algorithm>
+
+using namespace nrocm_adjoint;
 
 namespace {
 
@@ -284,176 +287,6 @@ __global__ __launch_bounds__(64) void getrf_getrs_batched_kernel(
     }
 }
 
-// x of lane T of the eight-lane group, in lane J (T, J static)
-template <int J, int T>
-__device__ __forceinline__ double from_lane(double x)
-{
-    if constexpr (J == T) {
-        return x;
-    } else {
-        constexpr int CTRL = J > T ? 0x110 + (J - T) : 0x100 + (T - J);  // row_shr, row_shl
-        const long long v = __double_as_longlong(x);
-        const int lo = __builtin_amdgcn_mov_dpp((int)v, CTRL, 0xf, 0xf, true);
-        const int hi = __builtin_amdgcn_mov_dpp((int)(v >> 32), CTRL, 0xf, 0xf, true);
-        return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-    }
-}
-
-// res + x of lanes FROM, FROM + STEP, ... (COUNT of them), in that order, in lane J
-template <int J, int FROM, int STEP, int COUNT>
-__device__ __forceinline__ double add_lanes(double res, double x)
-{
-    if constexpr (COUNT > 0) {
-        res += from_lane<J, FROM>(x);
-        res = add_lanes<J, FROM + STEP, STEP, COUNT - 1>(res, x);
-    }
-    return res;
-}
-
-// The adjoint's two substitutions read a matrix column by column; a group of
-// eight lanes holds one member, lane c the solved values of index c modulo 8:
-// the eight interleaved accumulators of dotx (src/base/blas.rs:93-167) are the
-// eight lanes.  The columns are fetched AHEAD steps before their use.
-constexpr int AHEAD = 4;
-
-template <int KM>
-struct Column {
-    double x[KM];  // the elements that meet solved blocks 0, 1, ...
-    double cur;    // those of the block in work
-};
-
-// ---- U^T y = g, i = 8 kb + J ascending: the products of whole blocks of 8
-// before i in the lanes' accumulators, those of i's own block one after another.
-template <int KM, int CH, int J>
-__device__ __forceinline__ void upper_step(int kb, int c, const Column<KM> &u, const double (&z)[CH][KM],
-                                           double (&cur)[CH], const double (&gv)[CH])
-{
-#pragma unroll
-    for (int q = 0; q < CH; ++q) {
-        double acc = 0.0;
-#pragma unroll
-        for (int k = 0; k < KM; ++k) {
-            const double p = u.x[k] * z[q][k];
-            acc += k < kb ? p : 0.0;
-        }
-        const double tail = u.cur * cur[q];
-        const double pair = acc + from_lane<0, 4>(acc);  // in lanes 0..3
-        double res = add_lanes<J, 0, 1, 4>(0.0, pair);
-        res = add_lanes<J, 0, 1, J>(res, tail);
-        const double y = (gv[q] - res) / u.cur;  // in lane J
-        cur[q] = c == J ? y : cur[q];
-    }
-}
-
-// accumulators 0..3 (each with its pair) of step J of the descending pass: T = 0..3
-template <int J, int T>
-__device__ __forceinline__ double add_pairs(double res, double pair)
-{
-    if constexpr (T < 4) {
-        res += from_lane<J, (J + 7 - T) & 3>(pair);
-        res = add_pairs<J, T + 1>(res, pair);
-    }
-    return res;
-}
-
-// ---- L^T z = y, i = n - 1 - s descending, s = 8 kb + J: counted from the end
-// (e = n - 1 - row), the dot runs over e = s - 1 down to 0, so its whole blocks
-// of 8 end at e = J and the tail is e = J - 1 .. 0.  Accumulator t holds the e
-// with e = J - 1 - t modulo 8.
-template <int KM, int CH, int J>
-__device__ __forceinline__ void lower_step(int kb, int c, const Column<KM> &l, const double (&z)[CH][KM],
-                                           double (&cur)[CH], const double (&yv)[CH])
-{
-#pragma unroll
-    for (int q = 0; q < CH; ++q) {
-        const double pc = l.cur * cur[q];
-        double acc = 0.0;
-        acc += (kb > 0 && c < J) ? pc : 0.0;
-        double p0 = 0.0;
-#pragma unroll
-        for (int k = KM - 1; k >= 0; --k) {
-            const double p = l.x[k] * z[q][k];
-            acc += (k < kb && (k > 0 || c >= J)) ? p : 0.0;
-            if (k == 0) p0 = p;
-        }
-        const double tail = kb > 0 ? p0 : pc;
-        const double pair = acc + from_lane<0, 4>(acc);  // in lanes 0..3
-        double res = add_pairs<J, 0>(0.0, pair);
-        res = add_lanes<J, J - 1, -1, J>(res, tail);
-        cur[q] = c == J ? yv[q] - res : cur[q];  // the unit diagonal divides by one
-    }
-}
-
-template <int KM>
-__device__ __forceinline__ void fetch_upper(Column<KM> &u, const double *M, int n, int i, int c)
-{
-    i = min(i, n - 1);
-    const double *col = M + (size_t)i * n;
-#pragma unroll
-    for (int k = 0; k < KM; ++k) u.x[k] = col[min(8 * k + c, i)];
-    u.cur = col[min((i & ~7) + c, i)];
-}
-
-template <int KM>
-__device__ __forceinline__ void fetch_lower(Column<KM> &l, const double *M, int n, int s, int c)
-{
-    s = min(s, n - 1);
-    const int i = n - 1 - s, top = min(i + 1, n - 1);
-    const double *col = M + (size_t)i * n;
-#pragma unroll
-    for (int k = 0; k < KM; ++k) l.x[k] = col[max(n - 1 - 8 * k - c, top)];
-    l.cur = col[max(n - 1 - (s & ~7) - c, top)];
-}
-
-template <int KM, int CH, bool UPPER, int J>
-__device__ __forceinline__ void block_steps(int kb, int c, Column<KM> (&ring)[AHEAD], const double *M, int n,
-                                            const double (&z)[CH][KM], double (&cur)[CH], const double (&gv)[CH])
-{
-    if constexpr (J < 8) {
-        if constexpr (UPPER) {
-            upper_step<KM, CH, J>(kb, c, ring[J % AHEAD], z, cur, gv);
-            fetch_upper<KM>(ring[J % AHEAD], M, n, 8 * kb + J + AHEAD, c);
-        } else {
-            lower_step<KM, CH, J>(kb, c, ring[J % AHEAD], z, cur, gv);
-            fetch_lower<KM>(ring[J % AHEAD], M, n, 8 * kb + J + AHEAD, c);
-        }
-        block_steps<KM, CH, UPPER, J + 1>(kb, c, ring, M, n, z, cur, gv);
-    }
-}
-
-// One substitution over v (the group's values by row, overwritten by the result).
-template <int KM, int CH, int LD, bool UPPER>
-__device__ __forceinline__ void substitute(const double *M, int n, int blocks, int c, double (*v)[LD])
-{
-    Column<KM> ring[AHEAD];
-#pragma unroll
-    for (int s = 0; s < AHEAD; ++s) {
-        if constexpr (UPPER) fetch_upper<KM>(ring[s], M, n, s, c);
-        else fetch_lower<KM>(ring[s], M, n, s, c);
-    }
-    double z[CH][KM];
-#pragma unroll
-    for (int q = 0; q < CH; ++q)
-#pragma unroll
-        for (int k = 0; k < KM; ++k) z[q][k] = 0.0;
-    for (int kb = 0; kb < blocks; ++kb) {
-        const int e = 8 * kb + c, row = UPPER ? e : n - 1 - e;
-        double gv[CH], cur[CH];
-#pragma unroll
-        for (int q = 0; q < CH; ++q) {
-            gv[q] = v[q][max(row, 0)];
-            cur[q] = 0.0;
-        }
-        block_steps<KM, CH, UPPER, 0>(kb, c, ring, M, n, z, cur, gv);
-#pragma unroll
-        for (int q = 0; q < CH; ++q) {
-#pragma unroll
-            for (int k = 0; k < KM; ++k) z[q][k] = k == kb ? cur[q] : z[q][k];
-            if (e < n) v[q][row] = cur[q];
-        }
-    }
-}
-
 // Adjoint of X = A^{-1} B from LU::new's packed factors and pivots:
 //   U^T y = g  (tr_solve_upper_triangular, solve.rs:255-276,411-440),
 //   L^T z = y  (tr_solve_lower_triangular on the unit L, solve.rs:232-253,379-409),
@@ -494,7 +327,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void ge
     const int blocks = __builtin_amdgcn_readfirstlane((most + 7) >> 3);
     if (blocks == 0) return;
     // a group without a member, or with an empty one, walks a 1 x 1 zero
-    const double *const LU = n > 0 ? LUptr[jm] : kZeroCellLU;
+    const Matrix LU = (Matrix)(n > 0 ? LUptr[jm] : kZeroCellLU);
     const int nm = max(n, 1);
     if (n > 0) {
         const int *const P = Pptr[jm];
@@ -506,9 +339,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void ge
 #pragma unroll
             for (int q = 0; q < CH; ++q) v[g][q][i] = c0 + q < nrhs ? dX[i + (size_t)(c0 + q) * n] : 0.0;
         __syncthreads();
-        substitute<KM, CH, LD, true>(LU, nm, blocks, c, v[g]);
+        substitute<UPPER, KM, CH, LD>(LU, nm, blocks, c, v[g]);
         __syncthreads();
-        substitute<KM, CH, LD, false>(LU, nm, blocks, c, v[g]);
+        substitute<UNIT_LOWER, KM, CH, LD>(LU, nm, blocks, c, v[g]);
         __syncthreads();
         // the swaps (i, ipiv[i]) in reverse order, a lane per right-hand side
         if (c < CH) {
