@@ -325,9 +325,10 @@ int nrocm_batch_create(nrocm_handle h, int count, const int *n_host, int nrhs, n
     }
     if (count > 0) {
         std::vector<int> blocks(count);
-        for (int j = 0; j < count; ++j) {
-            blocks[j] = (int)bt->row_blocks;
-            bt->row_blocks += (n_host[j] + 127LL) / 128;
+        unsigned before = 0;  // differences are what is used: may wrap
+        for (int i = 0; i < count; ++i) {
+            blocks[i] = (int)before;
+            before += (unsigned)((n_host[bt->order_host[i]] + 127LL) / 128);
         }
         if (hipMalloc(&bt->order_dev, sizeof(int) * 3 * (size_t)count) != hipSuccess) {
             nrocm_batch_destroy(bt);

@@ -108,10 +108,9 @@ struct nrocm_batch_s {
     std::vector<int> lanes[2];
     int *order_dev = nullptr;       // device copy of order_host
     int *n_dev = nullptr;           // device copy of n_host (caller order)
-    // Blocks of 128 rows before each member (caller order) and in all: where a
-    // least-squares member's reflectors lie in the workspace.
+    // Blocks of 128 rows before each member of `order`: where a least-squares
+    // member's reflectors lie in the workspace.
     int *blocks_dev = nullptr;
-    long long row_blocks = 0;
     // hipGraph replays of captured launch sequences, keyed by their arguments
     // (a bounded cache, oldest entry evicted first).
     struct GraphEntry {

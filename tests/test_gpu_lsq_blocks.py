@@ -50,3 +50,10 @@ def test_splits(nl, n, count):
     ms[:3] = [2 * n + 60, 128, 300]
     order = np.argsort(-ms, kind="stable")
     _check(nl, ms, n, 1.0, sorted({0, 1, 2, *order[:4].tolist(), *order[-4:].tolist()}))
+
+
+def test_more_systems_than_one_launch_holds(nl):
+    """The records of 250,000 systems exceed what one launch takes."""
+    ms = np.full(250000, 3, dtype=np.int32)
+    ms[[0, 123456, 249999]] = [300, 200, 129]
+    _check(nl, ms, 1, 1.0, [0, 1, 2, 123455, 123456, 123457, 200000, 233000, 234000, 249998, 249999])
