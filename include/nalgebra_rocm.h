@@ -63,6 +63,14 @@ int nrocm_create(nrocm_handle *handle);
 int nrocm_destroy(nrocm_handle handle);
 int nrocm_set_stream(nrocm_handle handle, void *hip_stream);
 int nrocm_get_stream(nrocm_handle handle, void **hip_stream);
+/* A call that is captured into a caller's graph (the handle's stream is under
+ * capture) and needs scratch gets a buffer of its own, which no other call uses:
+ * the graph may be replayed on any stream beside any other call.  These buffers
+ * stay until the handle is destroyed, or until this call, which waits for the
+ * device and frees them; the graphs captured before it must not be replayed
+ * again.  (One launch of a graph at a time: replays of the same graph that
+ * overlap share its buffer.) */
+int nrocm_free_graph_scratch(nrocm_handle handle);
 const char *nrocm_status_string(int status);
 const char *nrocm_last_error(nrocm_handle handle);
 int nrocm_version(void);

@@ -56,11 +56,19 @@ struct nrocm_handle_s {
         void *ptr = nullptr;
         size_t bytes = 0;
         hipStream_t stream = nullptr;  // of the last call that took it
-        bool captured = false;         // a caller's graph holds its address
     };
     Scratch ws[2];                  // NROCM_WS_MAIN, NROCM_WS_LU
     hipEvent_t ws_ev = nullptr;     // orders a call on another stream after the last
-    std::vector<void *> retired;    // outgrown scratch that a caller's graph may still use
+    std::vector<void *> retired;    // outgrown scratch that could not be waited for
+    // Scratch of captured calls (nrocm_free_graph_scratch).
+    struct GraphScratch {
+        unsigned long long capture;
+        hipStream_t stream;
+        int which;
+        size_t bytes;
+        void *ptr;
+    };
+    std::vector<GraphScratch> graph_ws;
     // Small device-side scalars (counters, flags, norms).
     void *small = nullptr;          // 4 KiB: int[0] Cholesky block info, ints from NROCM_SMALL_PLAN: LU row plan
     // Streams for independent launches that may run side by side (created on
@@ -130,8 +138,8 @@ int nrocm_fail(nrocm_handle h, int status, const char *msg);
 // Ensures at least `bytes` of scratch; synchronises the stream when it grows.
 // NROCM_WS_LU is the LU's own (other routines factor while they hold the main
 // one); it starts with NROCM_WS_LU_FIRST bytes, all that min(m, n) <= 64 needs.
-// On a stream under capture nothing is freed, and what the graph may hold stays
-// until the handle is destroyed.
+// On a stream under capture it is the graph's own, until the handle is destroyed
+// or nrocm_free_graph_scratch is called.
 enum { NROCM_WS_MAIN = 0, NROCM_WS_LU = 1 };
 constexpr size_t NROCM_WS_LU_FIRST = (size_t)16384 * 64 * 8 + 8192;
 int nrocm_workspace(nrocm_handle h, size_t bytes, void **ptr, int which = NROCM_WS_MAIN);

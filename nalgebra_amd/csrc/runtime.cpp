@@ -37,49 +37,69 @@ static int order_after_last_user(nrocm_handle h, nrocm_handle_s::Scratch &w)
     return NROCM_OK;
 }
 
+// Allocations are no part of a capture, but are not allowed beside one (this
+// thread's or another's) unless the thread says so.
+struct RelaxedCapture {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
+// Scratch of a call that is being captured: the graph may be replayed at any
+// time and on any stream, so no other call ever gets this buffer.  Calls of one
+// capture on one stream follow each other and share it.  (A graph does not say
+// when it dies: user objects retained by one are not released with it.)
+static int graph_workspace(nrocm_handle h, size_t bytes, void **ptr, int which)
+{
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    unsigned long long id = 0;
+    NROCM_CHECK_HIP(h, hipStreamGetCaptureInfo(h->stream, &cap, &id));
+    for (const auto &g : h->graph_ws)
+        if (g.capture == id && g.stream == h->stream && g.which == which && g.bytes >= bytes) {
+            *ptr = g.ptr;
+            return NROCM_OK;
+        }
+    nrocm_handle_s::GraphScratch g{id, h->stream, which, bytes, nullptr};
+    RelaxedCapture relaxed;
+    if (hipMalloc(&g.ptr, bytes) != hipSuccess) return nrocm_fail(h, NROCM_ERR_ALLOC, "workspace allocation failed");
+    h->graph_ws.push_back(g);
+    *ptr = g.ptr;
+    return NROCM_OK;
+}
+
 int nrocm_workspace(nrocm_handle h, size_t bytes, void **ptr, int which)
 {
     nrocm_handle_s::Scratch &w = h->ws[which];
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    bool beside = false;  // the legacy stream beside a capture: nothing may be waited for
     if (hipStreamIsCapturing(h->stream, &cap) != hipSuccess) {
-        (void)hipGetLastError();  // the legacy stream beside a capture
-        cap = hipStreamCaptureStatusActive;
+        (void)hipGetLastError();
+        beside = true;
     }
-    const bool capturing = cap != hipStreamCaptureStatusNone;
-    if (!capturing) {
+    if (!beside && cap != hipStreamCaptureStatusNone) return graph_workspace(h, bytes, ptr, which);
+    if (!beside) {
         const int s = order_after_last_user(h, w);
         if (s != NROCM_OK) return s;
     }
     if (bytes > w.bytes) {
-        // an allocation is no part of a capture, but is not allowed beside one
-        // unless the thread says so
-        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-        if (capturing) NROCM_CHECK_HIP(h, hipThreadExchangeStreamCaptureMode(&mode));
-        int status = NROCM_OK;
+        RelaxedCapture relaxed;
         if (w.ptr) {
-            if (capturing || w.captured) {
+            if (beside) {
                 h->retired.push_back(w.ptr);
             } else {
                 // Work already queued may still use the old buffer.
-                hipError_t e = hipStreamSynchronize(h->stream);
-                if (e == hipSuccess) e = hipFree(w.ptr);
-                if (e != hipSuccess) status = nrocm_fail_hip(h, e, "workspace release");
+                NROCM_CHECK_HIP(h, hipStreamSynchronize(h->stream));
+                NROCM_CHECK_HIP(h, hipFree(w.ptr));
             }
-            if (status == NROCM_OK) w = nrocm_handle_s::Scratch();
+            w = nrocm_handle_s::Scratch();
         }
         const size_t want = bytes + bytes / 4;
-        if (status == NROCM_OK) {
-            if (hipMalloc(&w.ptr, want) == hipSuccess) {
-                w.bytes = want;
-            } else {
-                w.ptr = nullptr;
-                status = nrocm_fail(h, NROCM_ERR_ALLOC, "workspace allocation failed");
-            }
+        if (hipMalloc(&w.ptr, want) != hipSuccess) {
+            w.ptr = nullptr;
+            return nrocm_fail(h, NROCM_ERR_ALLOC, "workspace allocation failed");
         }
-        if (capturing) (void)hipThreadExchangeStreamCaptureMode(&mode);
-        if (status != NROCM_OK) return status;
+        w.bytes = want;
     }
-    w.captured = w.captured || capturing;
     w.stream = h->stream;
     *ptr = w.ptr;
     return NROCM_OK;
@@ -170,6 +190,7 @@ int nrocm_destroy(nrocm_handle h)
     for (auto &w : h->ws)
         if (w.ptr) (void)hipFree(w.ptr);
     for (void *p : h->retired) (void)hipFree(p);
+    for (const auto &g : h->graph_ws) (void)hipFree(g.ptr);
     if (h->small) (void)hipFree(h->small);
     delete h;
     return NROCM_OK;
@@ -187,6 +208,15 @@ int nrocm_get_stream(nrocm_handle h, void **stream)
     if (!h) return -1;
     if (!stream) return -2;
     *stream = (void *)h->stream;
+    return NROCM_OK;
+}
+
+int nrocm_free_graph_scratch(nrocm_handle h)
+{
+    if (!h) return -1;
+    NROCM_CHECK_HIP(h, hipDeviceSynchronize());
+    for (const auto &g : h->graph_ws) NROCM_CHECK_HIP(h, hipFree(g.ptr));
+    h->graph_ws.clear();
     return NROCM_OK;
 }
 

@@ -1,0 +1,107 @@
+"""Captured calls own their scratch: graphs replayed on several streams beside
+each other and beside eager calls of the same handle give what each call gives
+alone."""
+import ctypes as C
+import gc
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _ptr(t):
+    return C.c_void_p(t.data_ptr())
+
+
+def _problem(kind, n, seed):
+    """(inputs, run): run(out) queues one call on torch's current stream."""
+    from nalgebra_amd._lib import lib
+    from nalgebra_amd.linalg import handle
+    rng = np.random.default_rng(seed)
+    a = rng.uniform(-1, 1, (n, n))
+    if kind == "chol":
+        a = a @ a.T / n + np.eye(n)
+    elif kind == "solve":
+        a = a / n + np.eye(n)
+    a = torch.from_numpy(np.asfortranarray(a).ravel(order="F").copy()).cuda()
+    b = torch.from_numpy(rng.uniform(-1, 1, n)).cuda()
+    piv = torch.arange(n, dtype=torch.int32, device="cuda").flip(0).contiguous()
+
+    def run(out):
+        x, ints = out
+        h = handle()
+        if kind == "solve":
+            x.copy_(b)
+            st = lib().nrocm_dgetrs(h, n, 1, _ptr(a), n, _ptr(piv), _ptr(x), n, _ptr(ints), 0)
+        else:
+            x.copy_(a)
+            if kind == "lu":
+                st = lib().nrocm_dgetrf(h, n, n, _ptr(x), n, _ptr(ints), C.c_void_p(ints.data_ptr() + 4 * n), 0)
+            else:
+                st = lib().nrocm_dpotrf(h, n, _ptr(x), n, _ptr(ints), 0)
+        assert st == 0
+    size = n if kind == "solve" else n * n
+    return run, (torch.empty(size, dtype=torch.float64, device="cuda"), torch.zeros(n + 1, dtype=torch.int32, device="cuda"))
+
+
+@pytest.mark.parametrize("kind,n", [("lu", 60), ("lu", 300), ("chol", 400), ("solve", 1100)])
+def test_replays_beside_each_other_and_eager_calls(nl, kind, n):
+    jobs = [_problem(kind, n, s) for s in range(3)]
+    want = []
+    for run, out in jobs:
+        run(out)
+        torch.cuda.synchronize()
+        want.append([t.clone() for t in out])
+    torch.cuda.synchronize()
+    graphs = []
+    for run, out in jobs[:2]:
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            run(out)
+        graphs.append(g)
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    for round_ in range(6):
+        for _, out in jobs:
+            for t in out:
+                t.zero_()
+        torch.cuda.synchronize()
+        for _ in range(4):
+            for k in range(2):
+                with torch.cuda.stream(streams[k]):
+                    graphs[k].replay()
+            with torch.cuda.stream(streams[2]):
+                jobs[2][0](jobs[2][1])
+        torch.cuda.synchronize()
+        for k in range(3):
+            for got, ref in zip(jobs[k][1], want[k]):
+                assert torch.equal(got, ref), (kind, round_, k)
+
+
+def test_graph_scratch_is_given_back(nl):
+    """What captured calls took is free again after nrocm_free_graph_scratch."""
+    from nalgebra_amd._lib import lib
+    L = lib()
+    h = C.c_void_p()
+    assert L.nrocm_create(C.byref(h)) == 0
+    n, calls = 1000, 40
+    s = torch.cuda.Stream()
+    assert L.nrocm_set_stream(h, s.cuda_stream) == 0
+    a = torch.rand(n * n, dtype=torch.float64, device="cuda")
+    ints = torch.zeros(n + 1, dtype=torch.int32, device="cuda")
+    torch.cuda.synchronize()
+    gc.collect()
+    torch.cuda.empty_cache()
+    free0 = torch.cuda.mem_get_info()[0]
+    for _ in range(calls):
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=s):
+            assert L.nrocm_dgetrf(h, n, n, _ptr(a), n, _ptr(ints), C.c_void_p(ints.data_ptr() + 4 * n), 0) == 0
+        del g
+    torch.cuda.synchronize()
+    assert free0 - torch.cuda.mem_get_info()[0] >= calls * n * n * 8
+    assert L.nrocm_free_graph_scratch(h) == 0
+    assert free0 - torch.cuda.mem_get_info()[0] < calls * n * n * 4
+    assert L.nrocm_free_graph_scratch(None) == -1
+    assert L.nrocm_destroy(h) == 0
