@@ -16,6 +16,7 @@
 // 4*(l/16)+v for the FP32/BF16 instructions, row l/16+4*v for the FP64 one
 // (measured on gfx950 with a one-wavefront probe).
 #pragma once
+#include "access_rules.hpp"
 #include "nrocm_internal.hpp"
 
 #include <hip/hip_bf16.h>
@@ -236,11 +237,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(gemm_waves<
     // the last column's end.  16-byte loads need no more than the element's
     // alignment (4095 x 3001 x 2047 f32, every leading dimension odd: 967 -> 420 us;
     // element loads and slower edge tiles before).
-    const bool a_inside = bm + BM <= m;
-    const long a_last = lda >= m ? (long)(k - 1) * lda + m - VN : -1;  // the last place of a 16-byte load
-
     auto fetch = [&](int k0) {
-        if (k0 + BK <= k && (a_inside || bm + BM - VN + (long)(k0 + BK - 1) * lda <= a_last)) {
+        if (nrocm_rules::gemm_wide_slice(m, k, lda, bm, BM, k0, BK)) {
 #pragma unroll
             for (int p = 0; p < NPA; ++p)
                 ra[p] = *(const V *)(A + (bm + ar) + (long)(k0 + ac + CPA * p) * lda);
