@@ -20,4 +20,14 @@ NROCM_RULE bool gemm_wide_slice(long m, long k, long lda, long bm, long tile, lo
     return k0 + bk <= k && (bm + tile <= m || (lda >= m && bm + tile + (k0 + bk - 1) * lda <= m + (k - 1) * lda));
 }
 
+// chol_dot_backward: the loading wavefronts make the products of phase p (row
+// n - 1 - p, elements x[n - p + e], e < p) for p = 0 .. dot_last_phase(n), whole
+// rounds of DOT_AHEAD phases that begin two phases ahead.  Element e reads row
+// dot_first_row + min(e, dot_last_element), a row of x also where the phase has no
+// such element (e >= p), none at all (p = 0) or is past the last row (p >= n).
+constexpr int DOT_AHEAD = 4;
+NROCM_RULE int dot_last_phase(int n) { return (n + DOT_AHEAD - 1) / DOT_AHEAD * DOT_AHEAD + 1; }
+NROCM_RULE int dot_first_row(int n, int p) { return p < n ? n - p : 0; }
+NROCM_RULE int dot_last_element(int n, int p) { return n - 1 - dot_first_row(n, p); }
+
 }  // namespace nrocm_rules

@@ -23,6 +23,7 @@
 //     block with the compiler's division.
 // CH right-hand sides share every load of M and interleave in the chain.
 #pragma once
+#include "access_rules.hpp"
 #include "exact_div.hpp"
 
 namespace nrocm_sweep {
@@ -397,7 +398,7 @@ __device__ __forceinline__ double row_shr1(double v)
 }
 
 constexpr int DOT_SLOTS = 3;
-constexpr int DOT_AHEAD = 4;  // columns in flight per loading wavefront
+constexpr int DOT_AHEAD = nrocm_rules::DOT_AHEAD;  // columns in flight per loading wavefront
 constexpr int DOT_U = 16;     // chain steps per group, read one group ahead
 constexpr int DOT_HEAD = 10;  // slot head: L_ii, its reciprocal, the eight tail products
 
@@ -436,11 +437,10 @@ __device__ __forceinline__ void chol_dot_backward(const double *__restrict__ L, 
             r.extra = col[w == 1 ? min(1 + (p & ~7) + (lane & 7), last) : 0];
         };
         auto put = [&](const Col &r, int p) {
-            const int i = n - 1 - p;
             const int full = p & ~7, lim = p < n ? dot_groups(p) * 8 * U : 0;
             double *s = slots + (p % DOT_SLOTS) * sstride;
-            const double *x = xs + (i + 1) * CH;
-            const int emax = max(p - 1, 0);
+            const double *x = xs + nrocm_rules::dot_first_row(n, p) * CH;
+            const int emax = nrocm_rules::dot_last_element(n, p);
             double f[NR][CH], ft[CH];
 #pragma unroll
             for (int k = 0; k < NR; ++k)
@@ -480,7 +480,7 @@ __device__ __forceinline__ void chol_dot_backward(const double *__restrict__ L, 
         for (int j = 0; j < DOT_AHEAD; ++j) fetch(reg[j], j + 2);
         lds_barrier();
 #pragma unroll 1
-        for (int p = 0; p < n; p += DOT_AHEAD) {
+        for (int p = 0; p < n; p += DOT_AHEAD) {  // put() up to nrocm_rules::dot_last_phase
 #pragma unroll
             for (int j = 0; j < DOT_AHEAD; ++j) {
                 put(reg[j], p + j + 2);

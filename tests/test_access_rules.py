@@ -39,3 +39,17 @@ def test_gemm_wide_slices_stay_inside(tmp_path):
                     }
             }
     if (wide == 0) return 2;""")
+
+
+def test_dot_phases_read_rows_of_x(tmp_path):
+    """Every element of every phase, the rounds that end past the last row too."""
+    _run(tmp_path, r"""
+    for (int n = 1; n <= 70; ++n)
+        for (int p = 0; p <= dot_last_phase(n); ++p)
+            for (int e = 0; e < 200; ++e) {
+                const int row = dot_first_row(n, p) + std::min(e, dot_last_element(n, p));
+                if (row < 0 || row >= n || (e < p && p < n && row != n - p + e)) {
+                    std::printf("n %d phase %d element %d: row %d\n", n, p, e, row);
+                    return 1;
+                }
+            }""")
