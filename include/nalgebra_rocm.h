@@ -71,6 +71,13 @@ int nrocm_get_stream(nrocm_handle handle, void **hip_stream);
  * again.  (One launch of a graph at a time: replays of the same graph that
  * overlap share its buffer.) */
 int nrocm_free_graph_scratch(nrocm_handle handle);
+/* The kernels that hand results from workgroup to workgroup poll for them a
+ * bounded number of times (the bounds are some seconds and more).  A wait that
+ * runs out shows: info = -1 from nrocm_dgetrf, nrocm_dgetrs and
+ * nrocm_dqr_rsolve, and NaN in the results of these and of nrocm_dgeqrf,
+ * nrocm_sgeqrf (diag too) and nrocm_dpotrs.  polls > 0 replaces the bounds of
+ * this handle's calls from now on, 0 restores them. */
+int nrocm_set_wait_limit(nrocm_handle handle, long polls);
 const char *nrocm_status_string(int status);
 const char *nrocm_last_error(nrocm_handle handle);
 int nrocm_version(void);
@@ -96,7 +103,8 @@ int nrocm_sgemm(nrocm_handle handle, size_t m, size_t k, size_t n, float alpha,
  * ipiv[i] (int32, 0-based) = pivot row chosen at step i (i when no swap;
  * LU's PermutationSequence holds the pairs (i, ipiv[i]) with ipiv[i] != i,
  * src/linalg/permutation_sequence.rs:84-93).  info[0] = 0, or 1 + the first
- * step whose column was entirely zero (nalgebra skips it, lu.rs:107-110).
+ * step whose column was entirely zero (nalgebra skips it, lu.rs:107-110), or
+ * -1 if an internal wait timed out (nrocm_set_wait_limit).
  * Shape of nalgebra-lapack's LUScalar::xgetrf (nalgebra-lapack/src/lu.rs:351-380). */
 int nrocm_dgetrf(nrocm_handle handle, int m, int n, double *a, int lda, int *ipiv,
                  int *info, int mode);
@@ -253,7 +261,8 @@ int nrocm_dqr_qmul(nrocm_handle handle, int m, int n, const double *qr, int lda,
 int nrocm_dqr_rmul(nrocm_handle handle, int m, int n, const double *qr, int lda,
                    const double *diag, int nrhs, double *b, int ldb);
 /* QR::solve_mut's upper solve (qr.rs:224-256) on the leading n x n block:
- * B (n x nrhs) <- R^{-1} B.  info[0] = 0 or 1 + index of a zero diag. */
+ * B (n x nrhs) <- R^{-1} B.  info[0] = 0 or 1 + index of a zero diag (or -1 if an
+ * internal wait timed out, n > 12,224). */
 int nrocm_dqr_rsolve(nrocm_handle handle, int n, const double *qr, int lda,
                      const double *diag, int nrhs, double *b, int ldb, int *info);
 

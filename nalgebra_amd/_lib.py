@@ -41,6 +41,7 @@ _PROTOS = {
     "nrocm_destroy": (_i, [_vp]),
     "nrocm_set_stream": (_i, [_vp, _vp]),
     "nrocm_get_stream": (_i, [_vp, C.POINTER(_vp)]),
+    "nrocm_set_wait_limit": (_i, [_vp, C.c_long]),
     "nrocm_free_graph_scratch": (_i, [_vp]),
     "nrocm_status_string": (C.c_char_p, [_i]),
     "nrocm_last_error": (C.c_char_p, [_vp]),

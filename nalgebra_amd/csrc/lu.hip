@@ -60,10 +60,10 @@ struct LuBuffer {
 
 template <typename T, typename G>
 hipError_t lu_columns_group(hipStream_t st, T *A, int lda, int m, int c0, int ncols, int kend, int *ipiv, int *info,
-                            LuBuffer<T> &b, int ticket)
+                            LuBuffer<T> &b, int ticket, long limit)
 {
     hipLaunchKernelGGL((lu_columns_kernel<T, G>), dim3(nrocm_cdiv(ncols, G::W)), dim3(G::CT), 0, st, A, lda, m, c0,
-                       ncols, kend, ipiv, info, b.V + (size_t)c0 * b.ldv, b.ldv, b.H + c0, b.tickets + ticket);
+                       ncols, kend, ipiv, info, b.V + (size_t)c0 * b.ldv, b.ldv, b.H + c0, b.tickets + ticket, limit);
     return hipGetLastError();
 }
 
@@ -88,9 +88,9 @@ hipError_t lu_left_group(hipStream_t st, T *A, int lda, int m, int c0, int kend,
 // Factors columns [c0, c0 + ncols) (those below kend) and brings them up to date.
 template <typename T>
 hipError_t lu_columns(hipStream_t st, T *A, int lda, int m, int c0, int ncols, int kend, int *ipiv, int *info,
-                      LuBuffer<T> &b, int ticket)
+                      LuBuffer<T> &b, int ticket, long limit)
 {
-    return LU_BY_ROWS(lu_columns_group, m - c0, st, A, lda, m, c0, ncols, kend, ipiv, info, b, ticket);
+    return LU_BY_ROWS(lu_columns_group, m - c0, st, A, lda, m, c0, ncols, kend, ipiv, info, b, ticket, limit);
 }
 
 // The L columns of all but the range's last group, their rows in final order.
@@ -165,7 +165,7 @@ int getrf_whole(nrocm_handle h, hipStream_t st, int m, int n, T *A, int lda, int
     LuBuffer<T> b(buf, m, n);
     const int mn = std::min(m, n);
     LU_TRY(b.clear(st));
-    LU_TRY(lu_columns<T>(st, A, lda, m, 0, n, mn, ipiv, info, b, 0));
+    LU_TRY(lu_columns<T>(st, A, lda, m, 0, n, mn, ipiv, info, b, 0, nrocm_wait_limit(h, COL_SPIN_LIMIT)));
     LU_TRY(lu_left<T>(st, A, lda, m, 0, mn, ipiv, b));
     return NROCM_OK;
 }
@@ -178,8 +178,9 @@ int getrf_panels(nrocm_handle h, hipStream_t st, int m, int n, T *A, int lda, in
     const int mn = std::min(m, n);
     const bool exact = trail == TRAIL_EXACT;
     constexpr int NB = 64;
+    const long limit = nrocm_wait_limit(h, COL_SPIN_LIMIT);
     LU_TRY(b.clear(st));
-    LU_TRY(lu_columns<T>(st, A, lda, m, 0, std::min(NB, mn), std::min(NB, mn), ipiv, info, b, 0));
+    LU_TRY(lu_columns<T>(st, A, lda, m, 0, std::min(NB, mn), std::min(NB, mn), ipiv, info, b, 0, limit));
     for (int j0 = 0; j0 < mn; j0 += NB) {
         const int nb = std::min(NB, mn - j0), j1 = j0 + nb;
         LU_TRY(lu_left<T>(st, A, lda, m, j0, j1, ipiv, b));
@@ -190,7 +191,7 @@ int getrf_panels(nrocm_handle h, hipStream_t st, int m, int n, T *A, int lda, in
             LU_TRY(trailing<T>(st, trail, A, lda, j1, m, j1, j2, j0, nb));
             const int s = nrocm_fork_on(h, st, 1);
             if (s != NROCM_OK) return s;
-            LU_TRY(lu_columns<T>(h->aux[0], A, lda, m, j1, j2 - j1, j2, ipiv, info, b, j1 / NB));
+            LU_TRY(lu_columns<T>(h->aux[0], A, lda, m, j1, j2 - j1, j2, ipiv, info, b, j1 / NB, limit));
         }
         LU_TRY(trailing<T>(st, trail, A, lda, j1, m, j2, n, j0, nb));
         if (j2 > j1) {
@@ -500,7 +501,7 @@ int getrf_graph(nrocm_handle h, int m, int n, T *A, int lda, int *ipiv, int *inf
     s = nrocm_aux_init(h);  // streams and events exist before the capture
     if (s != NROCM_OK) return s;
     const long long key[8] = {1000 + (long long)sizeof(T) + 16 * (long long)trail, (long long)m << 32 | n, lda,
-                              (long long)A, (long long)ipiv, (long long)info, (long long)buf, 0};
+                              (long long)A, (long long)ipiv, (long long)info, (long long)buf, h->wait_polls};
     return nrocm_graph_run(h, key, [&](hipStream_t st) {
         return getrf_panels<T>(h, st, m, n, A, lda, ipiv, info, trail, buf);
     });

@@ -18,7 +18,8 @@
 //   * a published element is its own flag (the buffer starts as a signalling
 //     NaN pattern; a value that is this very pattern is published quieted).
 // Group tickets are taken in column order, so the group that is waited for is
-// running.  Waits are bounded.
+// running.  Waits are bounded: a group that gives up takes NaN for what it waited
+// for and sets info to -1.
 // The range is the whole matrix up to WHOLE_ROWS rows (one launch instead of
 // some hundred: 500 x 500 2.45 -> 0.69 ms) and 64 columns above it (the
 // trailing matrix then takes rank-64 updates; 4096 x 4096 FAST 25.3 -> 13.3 ms).
@@ -45,7 +46,7 @@ using Group4K = Group<512, 8, 4>;
 using Group8K = Group<512, 16, 2>;
 using Group16K = Group<512, 32, 1>;
 constexpr int COLUMNS_ROWS_MAX = Group16K::ROWS;
-constexpr long COL_SPIN_LIMIT = 1L << 21;
+constexpr long COL_SPIN_LIMIT = 1L << 21;  // some seconds
 
 template <typename T> struct ColWord;
 template <> struct ColWord<double> {
@@ -117,7 +118,7 @@ __device__ __forceinline__ float uniform_lane63(float v)
 template <typename T, typename G>
 __global__ __launch_bounds__(G::CT) void lu_columns_kernel(T *A, int lda, int m, int c0, int ncols, int kend, int *ipiv,
                                                         int *info, typename ColWord<T>::U *V, int ldv,
-                                                        typename ColWord<T>::U *H, int *ticket)
+                                                        typename ColWord<T>::U *H, int *ticket, long limit)
 {
     typedef typename ColWord<T>::U U;
     constexpr U EMPTY = ColWord<T>::EMPTY;
@@ -169,6 +170,7 @@ __global__ __launch_bounds__(G::CT) void lu_columns_kernel(T *A, int lda, int m,
             }
         };
         long spins = 0;
+        bool lost = false;
         for (;;) {
             issue();
             bool ok = true;
@@ -178,8 +180,18 @@ __global__ __launch_bounds__(G::CT) void lu_columns_kernel(T *A, int lda, int m,
 #pragma unroll
                 for (int s = 0; s < RPT; ++s) ok = ok && w[s][k] != EMPTY;
             }
-            if (ok || ++spins > COL_SPIN_LIMIT) break;
+            lost = !ok && ++spins >= limit;
+            if (ok || lost) break;
             __builtin_amdgcn_s_sleep(1);
+        }
+        if (__builtin_expect(lost, 0)) {
+            __hip_atomic_store(info, -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+            for (int k = 0; k < W; ++k) {
+                hw[k] = hw[k] == EMPTY ? (U)(kh + k) : hw[k];  // no swap: positions stay valid
+#pragma unroll
+                for (int s = 0; s < RPT; ++s) w[s][k] = EMPTY | ColWord<T>::QUIET;
+            }
         }
         // the group's swaps
         unsigned skip = 0;
@@ -333,7 +345,8 @@ __global__ __launch_bounds__(G::CT) void lu_columns_kernel(T *A, int lda, int m,
                     }
                 }
             }
-            if (t == 0) piv_word[c] = zero ? (k | PIV_SKIP) : piv;
+            // (after a lost wait a position may be held by no row; what is published stays a row's)
+            if (t == 0) piv_word[c] = zero ? (k | PIV_SKIP) : piv < m ? piv : k;
             if (zero && first_zero == 0) first_zero = k + 1;
 #pragma unroll
             for (int s = 0; s < RPT; ++s)
@@ -352,6 +365,7 @@ __global__ __launch_bounds__(G::CT) void lu_columns_kernel(T *A, int lda, int m,
     }
     if (first_zero != 0 && t == 0) {  // the first such column of the matrix (after the loop: a load in it would
         // make every column wait for its own stores)
+        // a lost wait's -1 stays
         int seen = __hip_atomic_load(info, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         while ((seen == 0 || seen > first_zero) &&
                !__hip_atomic_compare_exchange_strong(info, &seen, first_zero, __ATOMIC_RELAXED, __ATOMIC_RELAXED,

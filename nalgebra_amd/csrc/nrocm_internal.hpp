@@ -94,7 +94,11 @@ struct nrocm_handle_s {
     // 1 when the last nrocm_dgesv_ir call replaced its windowed factors by
     // partial-pivoting factors.
     int ir_fallback = 0;
+    long wait_polls = 0;  // nrocm_set_wait_limit
 };
+
+// Polls after which a kernel's wait for another workgroup gives up.
+static inline long nrocm_wait_limit(nrocm_handle h, long usual) { return h->wait_polls > 0 ? h->wait_polls : usual; }
 
 // Runs `body(stream)` through the handle's graph cache: on a miss the launches
 // are captured into a new graph; either way the graph is launched on h->stream.

@@ -157,7 +157,8 @@ __global__ __launch_bounds__(256) void geqrf_exact_kernel(T *A, int m, int n, in
 //
 // A published element is its own flag: the buffer starts as a signalling NaN
 // pattern, which no arithmetic result has (results are quieted), and a reader
-// polls until another value is there.  Waits are bounded.
+// polls until another value is there.  Waits are bounded: a reader that gives up
+// goes on with that NaN, which reaches every later column and its diagonal entry.
 constexpr int PT = 512;               // threads per workgroup
 constexpr long QR_SPIN_LIMIT = 1L << 21;  // some seconds
 
@@ -268,8 +269,10 @@ __host__ __device__ constexpr int prod_stride(int m) { return (m + 31) / 32 * 32
 __host__ __device__ constexpr size_t qr_lds_elements(int m, int pc) { return (size_t)pc * prod_stride(m) + DOT_SLACK; }
 
 // Reflects columns KB..nc of x through axis v (rows j.., the thread's own)
-// with the given sign (reflect_with_sign, reflection.rs:70-83).  Every thread
-// of the workgroup calls it.
+// with the given sign (reflect_with_sign, reflection.rs:70-83), or, with a sign
+// of 0, leaves them.  Every thread of the workgroup calls it: whether there is an
+// axis is no reason to skip its barriers, because after a wait that ran out the
+// wavefronts may differ about it.
 template <typename T, int RPT, int PC, int KB>
 __device__ __forceinline__ void reflect(T (&x)[PC][RPT], const T (&v)[RPT], T sign, int j, int m, int nc, T *prod,
                                         T *fac)
@@ -298,7 +301,7 @@ __device__ __forceinline__ void reflect(T (&x)[PC][RPT], const T (&v)[RPT], T si
         for (int s = 0; s < RPT; ++s) {
             const int r = t + PT * s;
             const T y = axcpy1<T>(f, v[s], T(1), sign, x[c][s]);
-            x[c][s] = r >= j ? y : x[c][s];
+            x[c][s] = r >= j && sign != T(0) ? y : x[c][s];  // NaN reflects too
         }
     }
 }
@@ -412,7 +415,8 @@ __device__ __forceinline__ void own_columns(T (&x)[PC][RPT], int c0, int nc, int
 
 template <typename T, int RPT, int PC>
 __global__ __launch_bounds__(PT) void geqrf_columns_kernel(T *A, int m, int n, int lda, T *diag,
-                                                           typename Word<T>::U *V, typename Word<T>::U *H, int *ticket)
+                                                           typename Word<T>::U *V, typename Word<T>::U *H, int *ticket,
+                                                           long limit)
 {
     typedef typename Word<T>::U U;
     extern __shared__ __align__(16) unsigned char qr_lds[];
@@ -454,7 +458,7 @@ __global__ __launch_bounds__(PT) void geqrf_columns_kernel(T *A, int m, int n, i
 #pragma unroll
                 for (int s = 0; s < RPT; ++s) ok = ok && w[s] != Word<T>::EMPTY;
             }
-            if (ok || ++spins > QR_SPIN_LIMIT) break;
+            if (ok || ++spins >= limit) break;
             __builtin_amdgcn_s_sleep(1);
             issue(w, hw, j);
         }
@@ -463,7 +467,7 @@ __global__ __launch_bounds__(PT) void geqrf_columns_kernel(T *A, int m, int n, i
 #pragma unroll
         for (int s = 0; s < RPT; ++s) v[s] = Word<T>::value(w[s]);
         if (j + 1 < jend) issue(nw, nh, j + 1);
-        if (sign != T(0)) reflect<T, RPT, PC, 0>(x, v, sign, j, m, nc, prod, fac);
+        reflect<T, RPT, PC, 0>(x, v, sign, j, m, nc, prod, fac);
 #pragma unroll
         for (int s = 0; s < RPT; ++s) w[s] = nw[s];
         hw = nh;
@@ -601,7 +605,8 @@ int geqrf_columns(nrocm_handle h, int m, int n, T *a, int lda, T *diag)
     }
     nrocm_allow_lds<geqrf_columns_kernel<T, RPT, PC>>();
     hipLaunchKernelGGL((geqrf_columns_kernel<T, RPT, PC>), dim3(groups), dim3(PT),
-                       qr_lds_elements(m, PC) * sizeof(T), h->stream, a, m, n, lda, diag, V, H, ticket);
+                       qr_lds_elements(m, PC) * sizeof(T), h->stream, a, m, n, lda, diag, V, H, ticket,
+                       nrocm_wait_limit(h, QR_SPIN_LIMIT));
     NROCM_CHECK_LAUNCH(h);
     return NROCM_OK;
 }

@@ -211,6 +211,14 @@ int nrocm_get_stream(nrocm_handle h, void **stream)
     return NROCM_OK;
 }
 
+int nrocm_set_wait_limit(nrocm_handle h, long polls)
+{
+    if (!h) return -1;
+    if (polls < 0) return -2;
+    h->wait_polls = polls;
+    return NROCM_OK;
+}
+
 int nrocm_free_graph_scratch(nrocm_handle h)
 {
     if (!h) return -1;

@@ -16,8 +16,8 @@
 // (before: one wavefront per 64 rows, one right-hand side at a time, a load and a
 // lane mask in every step of the diagonal block).
 // The tag array is cleared at the start of every call and every launch of a
-// call has its own epoch.  Waits are bounded: a wait that runs out sets info
-// to -1 and the kernel still exits.
+// call has its own epoch.  Waits are bounded: a wait that runs out takes NaN for
+// the values, sets info to -1 (Cholesky has none) and the kernel still exits.
 #include "internal_launch.hpp"
 #include "solve_sweep.hpp"
 
@@ -33,7 +33,7 @@ constexpr int SUPER = SWEEP_WAVES * LB;   // rows per workgroup
 constexpr int PERM_LDS_MAX = 16384;       // composed permutation kept in LDS up to this n
 constexpr int PREP_WAVES = 16;
 constexpr int TICKETS = 60;               // launches per clearing of the header
-constexpr size_t HEADER_BYTES = 256;      // tickets, then the timeout word
+constexpr size_t HEADER_BYTES = 256;      // tickets
 
 typedef unsigned long long u64;
 
@@ -56,10 +56,11 @@ __device__ __forceinline__ double untag(u64 lo, u64 hi)
 }
 
 template <int CH>
-__device__ __forceinline__ void await(const u64 *src, unsigned epoch, double (&v)[CH], int *info)
+__device__ __forceinline__ void await(const u64 *src, unsigned epoch, double (&v)[CH], int *info, long limit)
 {
     u64 w[2 * CH];
     long spins = 0;
+    bool lost = false;
     for (;;) {
         bool ok = true;
 #pragma unroll
@@ -67,14 +68,15 @@ __device__ __forceinline__ void await(const u64 *src, unsigned epoch, double (&v
 #pragma unroll
         for (int c = 0; c < 2 * CH; ++c) ok = ok && (unsigned)(w[c] >> 32) == epoch;
         if (ok) break;
-        if (++spins > SPIN_LIMIT) {
-            atomicExch(info, -1);
+        if (++spins >= limit) {
+            lost = true;
+            if (info) atomicExch(info, -1);
             break;
         }
         __builtin_amdgcn_s_sleep(1);
     }
 #pragma unroll
-    for (int c = 0; c < CH; ++c) v[c] = untag(w[2 * c], w[2 * c + 1]);
+    for (int c = 0; c < CH; ++c) v[c] = lost ? __builtin_nan("") : untag(w[2 * c], w[2 * c + 1]);
 }
 
 // One sweep of a large solve.  LU_FWD reads b through perm and publishes y;
@@ -85,7 +87,7 @@ __global__ __launch_bounds__(THREADS) void sweep_lookback_kernel(const double *_
                                                                  const double *__restrict__ dg,
                                                                  const int *__restrict__ perm, double *B, int ldb,
                                                                  int nrhs, int ngroups, int *ticket, u64 *tags,
-                                                                 unsigned epoch_in, unsigned epoch, int *info)
+                                                                 unsigned epoch_in, unsigned epoch, int *info, long limit)
 {
     __shared__ __align__(16) double D[DSLOTS * LB * LB];
     __shared__ __align__(16) double xs[SUPER * CH];               // this workgroup's blocks
@@ -127,7 +129,7 @@ __global__ __launch_bounds__(THREADS) void sweep_lookback_kernel(const double *_
         // a finished block is never the matrix's last one: it is full
         const int u = J * LB + lane;
         double v[CH];
-        await<CH>(gtags + (size_t)(from_top(KIND) ? u : n - 1 - u) * CH * 2, epoch, v, info);
+        await<CH>(gtags + (size_t)(from_top(KIND) ? u : n - 1 - u) * CH * 2, epoch, v, info, limit);
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
         for (int c = 0; c < CH; ++c) xw[w][lane * CH + c] = v[c];
@@ -287,7 +289,7 @@ struct Sweeps {
         const unsigned in = epoch++;
         hipLaunchKernelGGL((sweep_lookback_kernel<EXACT, KIND, CH>), dim3(nrocm_cdiv(n, SUPER) * ngroups),
                            dim3(THREADS), 0, st, M, lda, n, dg, perm, B, ldb, cols, ngroups, ticket + in % TICKETS,
-                           tags, in, epoch, info);
+                           tags, in, epoch, info, nrocm_wait_limit(h, SPIN_LIMIT));
         NROCM_CHECK_LAUNCH(h);
         return NROCM_OK;
     }
@@ -350,7 +352,6 @@ int solve(nrocm_handle h, hipStream_t st, int n, int nrhs, const double *M, int 
     int *header = (int *)base;
     int *perm = (int *)(base + HEADER_BYTES);
     u64 *tags = (u64 *)(base + HEADER_BYTES + perm_bytes(n));
-    if (!info) info = header + TICKETS;  // a wait that ran out (never expected)
     Sweeps s{h, st, M, lda, n, dg, perm, header, tags, info};
     const int ch = std::min(cols == 1 ? 1 : cols == 2 ? 2 : 4, rhs_per_group(h->num_cus, std::min(cols, nrhs), nrocm_cdiv(n, SUPER)));
     for (int c0 = 0; c0 == 0 || c0 < nrhs; c0 += cols) {
@@ -363,7 +364,7 @@ int solve(nrocm_handle h, hipStream_t st, int n, int nrhs, const double *M, int 
         nrocm_allow_lds<prep_kernel>();
         hipLaunchKernelGGL(prep_kernel, dim3(blocks), dim3(PREP_WAVES * 64),
                            piv && n <= PERM_LDS_MAX ? (size_t)n * sizeof(int) : 0, st, tags, ntag, header, info,
-                           c0 == 0 && info != header + TICKETS, piv, n, perm);
+                           c0 == 0 && info, piv, n, perm);
         NROCM_CHECK_LAUNCH(h);
         if (n == 0) return NROCM_OK;
         if (cc <= 0) {  // no right-hand sides: only the diagonal is looked at
