@@ -273,8 +273,8 @@ int nrocm_dqr_rsolve(nrocm_handle handle, int n, const double *qr, int lda,
  * x = R^{-1} (Q^T b)[0..n), then `refine` FP64 residual-refinement
  * steps x += R^{-1} (Q^T (b - A x))[0..n) with b - A x formed in FP64.  A_j and
  * b_j are not modified; x is n x count f64 (column j = system j); info[j] = 0 or
- * 1 + index of a zero R diagonal (so also where all squares of a column underflow in
- * FP32).  The workspace is bounded: at most 2 GiB of reflectors at a time.  Replaces the tall solve nalgebra-lapack's
+ * 1 + index of a zero R diagonal.  A system with NaN or infinities gives NaN.
+ * The workspace is bounded: at most 2 GiB of reflectors at a time.  Replaces the tall solve nalgebra-lapack's
  * QrDecomposition::solve provides (nalgebra-lapack/src/qr/abstraction.rs:48-77,
  * qr_util.rs:167-230: ormqr then trtrs); core nalgebra's QR::solve is square-only
  * (src/linalg/qr.rs:214-217). */

@@ -7,7 +7,7 @@
 //    reflection_axis_mut (householder.rs:19-53) -> reflect_with_sign
 //    (src/geometry/reflection.rs:70-83).  Every dot product uses dotx's eight
 //    accumulators (src/base/blas.rs:93-167): independent chains, one lane each.
-// 2. Batched tall least squares (nrocm_sgels_batched): see qr_batched below.
+// 2. Batched tall least squares (nrocm_sgels_batched): qr_batched.inc.
 #include "gemm_kernels.hpp"
 #include "internal_launch.hpp"
 #include "solve_sweep.hpp"
@@ -677,18 +677,6 @@ __global__ void copy_cols_kernel(const double *B, int ldb, int n, int nrhs, doub
 }  // namespace
 
 // ---------------------------------------------------------------- batched tall least squares
-//
-// Per system (one 256-thread workgroup), with [A | b] copied into an f32
-// workspace W (m x (n+1)) so that A stays intact for the FP64 residual:
-//   for each 16-column block J:
-//     panel:    unblocked Householder (LAPACK larfg convention, v(0) = 1) on
-//               W[16J.., 16J..16J+16) held in registers, R block and V written
-//               back, T (16 x 16 upper, compact WY) from V^T V and tau
-//     trailing: C = W[16J.., 16J+16..n] (b included) <- (I - V T V^T)^T C
-//               computed as Wt = V^T C and C -= V (T^T Wt), both on
-//               v_mfma_f32_16x16x4f32 with 64-row chunks staged through LDS
-//   x0 = R^{-1} (Q^T b)[0..n)                      (f32 R, f64 arithmetic)
-//   refine: r = b - A x0 (FP64), x = x0 + R^{-1} (Q^T r)[0..n)
 #include "qr_batched.inc"
 
 extern "C" {
