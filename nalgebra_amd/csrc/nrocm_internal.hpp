@@ -45,19 +45,27 @@ void nrocm_allow_lds()
 
 constexpr int NROCM_SMALL_PLAN = 256;  // int offset of the LU row plan (257 ints) in small
 
+constexpr int NROCM_WS_STREAMS = 4;                     // as many as run side by side on the hardware's queues
+constexpr size_t NROCM_WS_OWN_BYTES = (size_t)64 << 20;  // calls with more fill the chip by themselves
+
 struct nrocm_handle_s {
     hipStream_t stream = nullptr;   // caller's stream (nullptr = legacy default stream)
     int device = 0;
     int num_cus = 0;
     std::string last_error;
 
-    // Growable scratch on the device, reused across calls (ordered on `stream`).
+    // Growable scratch on the device, reused across calls: up to
+    // NROCM_WS_OWN_BYTES one for each of NROCM_WS_STREAMS streams, so that calls on
+    // several streams run side by side, above that one for all.  A call on another
+    // stream than the last one's is ordered after it.
     struct Scratch {
         void *ptr = nullptr;
         size_t bytes = 0;
         hipStream_t stream = nullptr;  // of the last call that took it
+        unsigned long long used = 0;   // when, in calls; 0: never
     };
-    Scratch ws[2];                  // NROCM_WS_MAIN, NROCM_WS_LU
+    Scratch ws[2][NROCM_WS_STREAMS + 1];  // NROCM_WS_MAIN, NROCM_WS_LU
+    unsigned long long ws_clock = 0;
     hipEvent_t ws_ev = nullptr;     // orders a call on another stream after the last
     std::vector<void *> retired;    // outgrown scratch that could not be waited for
     // Scratch of captured calls (nrocm_free_graph_scratch).
@@ -141,11 +149,9 @@ int nrocm_fail_hip(nrocm_handle h, hipError_t e, const char *what);
 int nrocm_fail(nrocm_handle h, int status, const char *msg);
 // Ensures at least `bytes` of scratch; synchronises the stream when it grows.
 // NROCM_WS_LU is the LU's own (other routines factor while they hold the main
-// one); it starts with NROCM_WS_LU_FIRST bytes, all that min(m, n) <= 64 needs.
-// On a stream under capture it is the graph's own, until the handle is destroyed
-// or nrocm_free_graph_scratch is called.
+// one).  On a stream under capture it is the graph's own, until the handle is
+// destroyed or nrocm_free_graph_scratch is called.
 enum { NROCM_WS_MAIN = 0, NROCM_WS_LU = 1 };
-constexpr size_t NROCM_WS_LU_FIRST = (size_t)16384 * 64 * 8 + 8192;
 int nrocm_workspace(nrocm_handle h, size_t bytes, void **ptr, int which = NROCM_WS_MAIN);
 // Forks the handle's auxiliary streams from its stream (nrocm_fork) and joins
 // them back (nrocm_join): work launched on aux[i] in between runs concurrently

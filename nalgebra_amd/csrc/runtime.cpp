@@ -2,6 +2,7 @@
 // generators of libnalgebra_rocm.
 #include "nrocm_internal.hpp"
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 
@@ -67,9 +68,22 @@ static int graph_workspace(nrocm_handle h, size_t bytes, void **ptr, int which)
     return NROCM_OK;
 }
 
+// The scratch of this call's stream, or the one that all streams share for large
+// requests; with more streams than entries, that of the longest unused stream.
+static nrocm_handle_s::Scratch &scratch_of(nrocm_handle h, size_t bytes, int which)
+{
+    nrocm_handle_s::Scratch *const ws = h->ws[which];
+    if (bytes > NROCM_WS_OWN_BYTES) return ws[NROCM_WS_STREAMS];
+    int at = 0;
+    for (int i = 0; i < NROCM_WS_STREAMS; ++i) {
+        if (ws[i].used != 0 && ws[i].stream == h->stream) return ws[i];
+        if (ws[i].used < ws[at].used) at = i;
+    }
+    return ws[at];
+}
+
 int nrocm_workspace(nrocm_handle h, size_t bytes, void **ptr, int which)
 {
-    nrocm_handle_s::Scratch &w = h->ws[which];
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     bool beside = false;  // the legacy stream beside a capture: nothing may be waited for
     if (hipStreamIsCapturing(h->stream, &cap) != hipSuccess) {
@@ -77,6 +91,7 @@ int nrocm_workspace(nrocm_handle h, size_t bytes, void **ptr, int which)
         beside = true;
     }
     if (!beside && cap != hipStreamCaptureStatusNone) return graph_workspace(h, bytes, ptr, which);
+    nrocm_handle_s::Scratch &w = scratch_of(h, bytes, which);
     if (!beside) {
         const int s = order_after_last_user(h, w);
         if (s != NROCM_OK) return s;
@@ -93,7 +108,7 @@ int nrocm_workspace(nrocm_handle h, size_t bytes, void **ptr, int which)
             }
             w = nrocm_handle_s::Scratch();
         }
-        const size_t want = bytes + bytes / 4;
+        const size_t want = bytes + std::min(bytes / 4, NROCM_WS_OWN_BYTES);
         if (hipMalloc(&w.ptr, want) != hipSuccess) {
             w.ptr = nullptr;
             return nrocm_fail(h, NROCM_ERR_ALLOC, "workspace allocation failed");
@@ -101,6 +116,7 @@ int nrocm_workspace(nrocm_handle h, size_t bytes, void **ptr, int which)
         w.bytes = want;
     }
     w.stream = h->stream;
+    w.used = ++h->ws_clock;
     *ptr = w.ptr;
     return NROCM_OK;
 }
@@ -161,13 +177,6 @@ int nrocm_create(nrocm_handle *handle)
         delete h;
         return NROCM_ERR_ALLOC;
     }
-    nrocm_handle_s::Scratch &lu = h->ws[NROCM_WS_LU];
-    if (hipMalloc(&lu.ptr, NROCM_WS_LU_FIRST) != hipSuccess) {
-        (void)hipFree(h->small);
-        delete h;
-        return NROCM_ERR_ALLOC;
-    }
-    lu.bytes = NROCM_WS_LU_FIRST;
     *handle = h;
     return NROCM_OK;
 }
@@ -187,8 +196,9 @@ int nrocm_destroy(nrocm_handle h)
     }
     if (h->fork_ev) (void)hipEventDestroy(h->fork_ev);
     if (h->ws_ev) (void)hipEventDestroy(h->ws_ev);
-    for (auto &w : h->ws)
-        if (w.ptr) (void)hipFree(w.ptr);
+    for (auto &kind : h->ws)
+        for (auto &w : kind)
+            if (w.ptr) (void)hipFree(w.ptr);
     for (void *p : h->retired) (void)hipFree(p);
     for (const auto &g : h->graph_ws) (void)hipFree(g.ptr);
     if (h->small) (void)hipFree(h->small);
