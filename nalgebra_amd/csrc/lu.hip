@@ -27,33 +27,35 @@ namespace {
 // 2.97 and 2.51, 2048 8.2 and 5.3).
 constexpr int WHOLE_ROWS = 1024;
 
-// Words of the pipeline's buffer for an m x n matrix: L columns and pivots,
-// after a header of one ticket per panel.
+// The pipeline's buffer, after a header of one ticket per panel: L columns and
+// pivots of all columns where the matrix is one range, else of two panels in turn
+// (lu_left_kernel, which has read the one, clears the other for the next panel).
 constexpr size_t LU_HEADER_BYTES = 2048;
-template <typename T>
-size_t lu_buffer_bytes(int m, int n)
-{
-    const size_t mn = (size_t)std::min(m, n);
-    return LU_HEADER_BYTES + (mn * m + mn) * sizeof(typename ColWord<T>::U);
-}
+constexpr int LU_NB = 64;  // columns of a panel
+
+bool lu_is_whole(int m, int n) { return m <= WHOLE_ROWS || std::min(m, n) <= LU_NB; }
 
 template <typename T>
 struct LuBuffer {
     typedef typename ColWord<T>::U U;
     int *tickets;
-    U *V, *H;
-    int ldv;
-    size_t words;
+    U *words;
+    int ldv, cols, parts;
 
     LuBuffer(void *p, int m, int n)
-        : tickets((int *)p), V((U *)((char *)p + LU_HEADER_BYTES)), H(V + (size_t)std::min(m, n) * m), ldv(m),
-          words((size_t)std::min(m, n) * m + std::min(m, n))
+        : tickets((int *)p), words((U *)((char *)p + LU_HEADER_BYTES)), ldv(m),
+          cols(lu_is_whole(m, n) ? std::min(m, n) : LU_NB), parts(lu_is_whole(m, n) ? 1 : 2)
     {
     }
-    hipError_t clear(hipStream_t st)
+    size_t part_words() const { return (size_t)cols * ldv + cols; }
+    size_t bytes() const { return LU_HEADER_BYTES + parts * part_words() * sizeof(U); }
+    U *V(int c0) const { return words + (size_t)(c0 / LU_NB % parts) * part_words(); }
+    U *H(int c0) const { return V(c0) + (size_t)cols * ldv; }
+    hipError_t clear(hipStream_t st)  // the first part
     {
-        hipLaunchKernelGGL((fill_words_kernel<U>), dim3(std::min<size_t>(4096, nrocm_cdiv(words, 1024) + 4)), dim3(256),
-                           0, st, V, words, ColWord<T>::EMPTY, tickets, (int)(LU_HEADER_BYTES / sizeof(int)));
+        const size_t count = part_words();
+        hipLaunchKernelGGL((fill_words_kernel<U>), dim3(std::min<size_t>(4096, nrocm_cdiv(count, 1024) + 4)), dim3(256),
+                           0, st, words, count, ColWord<T>::EMPTY, tickets, (int)(LU_HEADER_BYTES / sizeof(int)));
         return hipGetLastError();
     }
 };
@@ -63,17 +65,19 @@ hipError_t lu_columns_group(hipStream_t st, T *A, int lda, int m, int c0, int nc
                             LuBuffer<T> &b, int ticket, long limit)
 {
     hipLaunchKernelGGL((lu_columns_kernel<T, G>), dim3(nrocm_cdiv(ncols, G::W)), dim3(G::CT), 0, st, A, lda, m, c0,
-                       ncols, kend, ipiv, info, b.V + (size_t)c0 * b.ldv, b.ldv, b.H + c0, b.tickets + ticket, limit);
+                       ncols, kend, ipiv, info, b.V(c0), b.ldv, b.H(c0), b.tickets + ticket, limit);
     return hipGetLastError();
 }
 
 template <typename T, typename G>
-hipError_t lu_left_group(hipStream_t st, T *A, int lda, int m, int c0, int kend, const int *ipiv, LuBuffer<T> &b)
+hipError_t lu_left_group(hipStream_t st, T *A, int lda, int m, int c0, int kend, const int *ipiv, LuBuffer<T> &b,
+                         bool next)
 {
     const int groups = (int)nrocm_cdiv(kend - c0, G::W);
     if (groups > 1 && m > c0 + G::W)
         hipLaunchKernelGGL((lu_left_kernel<T, G::W>), dim3(nrocm_cdiv(m - c0 - G::W, 256), groups - 1), dim3(256), 0,
-                           st, A, lda, m, c0, kend, ipiv, b.V + (size_t)c0 * b.ldv, b.ldv);
+                           st, A, lda, m, c0, kend, ipiv, b.V(c0), b.ldv, next ? b.V(kend) : nullptr,
+                           next ? b.H(kend) : nullptr);
     return hipGetLastError();
 }
 
@@ -93,11 +97,12 @@ hipError_t lu_columns(hipStream_t st, T *A, int lda, int m, int c0, int ncols, i
     return LU_BY_ROWS(lu_columns_group, m - c0, st, A, lda, m, c0, ncols, kend, ipiv, info, b, ticket, limit);
 }
 
-// The L columns of all but the range's last group, their rows in final order.
+// The L columns of all but the range's last group, their rows in final order; with
+// `next`, a full panel with another one after it, also clears that one's part.
 template <typename T>
-hipError_t lu_left(hipStream_t st, T *A, int lda, int m, int c0, int kend, const int *ipiv, LuBuffer<T> &b)
+hipError_t lu_left(hipStream_t st, T *A, int lda, int m, int c0, int kend, const int *ipiv, LuBuffer<T> &b, bool next)
 {
-    return LU_BY_ROWS(lu_left_group, m - c0, st, A, lda, m, c0, kend, ipiv, b);
+    return LU_BY_ROWS(lu_left_group, m - c0, st, A, lda, m, c0, kend, ipiv, b, next);
 }
 
 template <typename T>
@@ -166,7 +171,7 @@ int getrf_whole(nrocm_handle h, hipStream_t st, int m, int n, T *A, int lda, int
     const int mn = std::min(m, n);
     LU_TRY(b.clear(st));
     LU_TRY(lu_columns<T>(st, A, lda, m, 0, n, mn, ipiv, info, b, 0, nrocm_wait_limit(h, COL_SPIN_LIMIT)));
-    LU_TRY(lu_left<T>(st, A, lda, m, 0, mn, ipiv, b));
+    LU_TRY(lu_left<T>(st, A, lda, m, 0, mn, ipiv, b, false));
     return NROCM_OK;
 }
 
@@ -177,13 +182,13 @@ int getrf_panels(nrocm_handle h, hipStream_t st, int m, int n, T *A, int lda, in
     LuBuffer<T> b(buf, m, n);
     const int mn = std::min(m, n);
     const bool exact = trail == TRAIL_EXACT;
-    constexpr int NB = 64;
+    constexpr int NB = LU_NB;
     const long limit = nrocm_wait_limit(h, COL_SPIN_LIMIT);
     LU_TRY(b.clear(st));
     LU_TRY(lu_columns<T>(st, A, lda, m, 0, std::min(NB, mn), std::min(NB, mn), ipiv, info, b, 0, limit));
     for (int j0 = 0; j0 < mn; j0 += NB) {
         const int nb = std::min(NB, mn - j0), j1 = j0 + nb;
-        LU_TRY(lu_left<T>(st, A, lda, m, j0, j1, ipiv, b));
+        LU_TRY(lu_left<T>(st, A, lda, m, j0, j1, ipiv, b, j1 < mn));
         LU_TRY(swap_rows<T>(st, A, lda, m, ipiv, j0, nb, 0, j0, j1, n));
         if (j1 < n) LU_TRY(trsm<T>(st, A, lda, j0, nb, j1, n, exact));
         const int j2 = j1 < mn ? std::min(mn, j1 + NB) : j1;  // the next panel
@@ -493,11 +498,11 @@ int getrf_graph(nrocm_handle h, int m, int n, T *A, int lda, int *ipiv, int *inf
     }
     if (m > COLUMNS_ROWS_MAX) return nrocm_fail(h, NROCM_ERR_UNSUPPORTED, "getrf: more than 16384 rows");
     void *buf = nullptr;
-    int s = nrocm_workspace(h, lu_buffer_bytes<T>(m, n), &buf, NROCM_WS_LU);
+    int s = nrocm_workspace(h, LuBuffer<T>(nullptr, m, n).bytes(), &buf, NROCM_WS_LU);
     if (s != NROCM_OK) return s;
     hipLaunchKernelGGL(fill_int_kernel, dim3(1), dim3(64), 0, h->stream, info, 1, 0);
     NROCM_CHECK_LAUNCH(h);
-    if (m <= WHOLE_ROWS || std::min(m, n) <= 64) return getrf_whole<T>(h, h->stream, m, n, A, lda, ipiv, info, buf);
+    if (lu_is_whole(m, n)) return getrf_whole<T>(h, h->stream, m, n, A, lda, ipiv, info, buf);
     s = nrocm_aux_init(h);  // streams and events exist before the capture
     if (s != NROCM_OK) return s;
     const long long key[8] = {1000 + (long long)sizeof(T) + 16 * (long long)trail, (long long)m << 32 | n, lda,

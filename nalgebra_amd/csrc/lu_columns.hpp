@@ -390,11 +390,20 @@ __global__ __launch_bounds__(G::CT) void lu_columns_kernel(T *A, int lda, int m,
 // Rows below group h = blockIdx.y of a factored range (all groups but the
 // last): position x of the final matrix holds what was at `who` when the group
 // started, which the range's swaps from there on, followed backwards, give.
+// nextV, nextH (or null): what the next panel, columns kend.., publishes into.
 template <typename T, int W>
 __global__ __launch_bounds__(256) void lu_left_kernel(T *A, int lda, int m, int c0, int kend,
                                                       const int *__restrict__ ipiv,
-                                                      const typename ColWord<T>::U *__restrict__ V, int ldv)
+                                                      const typename ColWord<T>::U *__restrict__ V, int ldv,
+                                                      typename ColWord<T>::U *__restrict__ nextV,
+                                                      typename ColWord<T>::U *__restrict__ nextH)
 {
+    if (nextV) {  // 64 columns, rows kend..m
+        const int row = kend + blockIdx.x * 256 + threadIdx.x;
+        if (row < m)
+            for (int c = blockIdx.y; c < 64; c += gridDim.y) nextV[(size_t)c * ldv + row] = ColWord<T>::EMPTY;
+        if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < 64) nextH[threadIdx.x] = ColWord<T>::EMPTY;
+    }
     const int k0 = c0 + blockIdx.y * W;
     const int x = k0 + W + blockIdx.x * 256 + threadIdx.x;
     const int lane = threadIdx.x & 63;
