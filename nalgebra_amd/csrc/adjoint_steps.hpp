@@ -30,6 +30,19 @@ __device__ __forceinline__ double add_lanes(double res, double x)
     return res;
 }
 
+// Members per wavefront of a batch: as few as fill the chip with one wavefront per
+// SIMD.  A step takes as long for one member as for eight, but its columns come
+// sooner, and the outer product is the whole wavefront's, member after member.
+// (Cholesky's adjoint, us, 8 in each wavefront, now, and with two per SIMD: 8 members
+// of 64, 4 right-hand sides 236 / 107 / 107, 512 of 64 246 / 113 / 112, 2048 of 16, one
+// 15.4 / 11.4 / 16.2, 4096 of 32 40.0 / 30.7 / 35.4.)
+inline int members_per_wave(int num_cus, int count)
+{
+    for (int per = 1; per < 8; per *= 2)
+        if ((long)count <= (long)per * 4 * num_cus) return per;
+    return 8;
+}
+
 // The adjoint's two substitutions read a matrix column by column; a group of
 // eight lanes holds one member, lane c the solved values of index c modulo 8:
 // the eight interleaved accumulators of dotx (src/base/blas.rs:93-167) are the

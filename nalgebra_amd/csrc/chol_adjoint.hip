@@ -6,10 +6,10 @@
 //   in order.
 //
 // Bound by the chains of the two substitutions, a division and a broadcast or a
-// dot per row: eight members share a wavefront, eight lanes each, no step needs a
-// barrier, and members of all sizes run in one launch, the largest first.  Before,
+// dot per row: up to eight members share a wavefront, eight lanes each, no step needs
+// a barrier, and members of all sizes run in one launch, the largest first.  Before,
 // a member had 16 to 64 lanes, a step one to three barriers and each range of
-// sizes its own launch: 4096 members of n = 32, one right-hand side, 92 -> 40 us,
+// sizes its own launch: 4096 members of n = 32, one right-hand side, 90 -> 31 us,
 // where reading L and X and writing dA take 10.
 #include "adjoint_steps.hpp"
 #include "internal_launch.hpp"
@@ -23,7 +23,8 @@ __device__ const double kZeroCell[1] = {0.0};
 // KM: blocks of 8 rows that a lane can hold; CH: right-hand sides at a time.
 template <int KM, int CH>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void potrs_backward_kernel(
-    const int *__restrict__ order, int count, const int *__restrict__ nsz, const double *const *__restrict__ Lptr,
+    const int *__restrict__ order, int count, int per, const int *__restrict__ nsz,
+    const double *const *__restrict__ Lptr,
     const double *const *__restrict__ Xptr, const double *const *__restrict__ dXptr,
     double *const *__restrict__ dAptr, double *const *__restrict__ dBptr, int nrhs)
 {
@@ -32,8 +33,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void po
     __shared__ double xs[8][CH][LD];  // the chunk of X
     const int lane = threadIdx.x;
     const int g = lane >> 3, c = lane & 7;
-    const int item = (int)blockIdx.x * 8 + g;
-    const bool valid = item < count;
+    const int item = (int)blockIdx.x * per + g;
+    const bool valid = g < per && item < count;
     const int jm = valid ? order[item] : 0;
     const int n = valid ? nsz[jm] : 0;
     int most = n;
@@ -75,7 +76,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void po
         // dA[r, k] = -1/2 (Lambda_r X_k + X_r Lambda_k), the whole wavefront on one
         // member at a time, along its columns
 #pragma unroll 1
-        for (int m = 0; m < 8; ++m) {
+        for (int m = 0; m < per; ++m) {
             const int mn = __builtin_amdgcn_readlane(n, 8 * m);
             if (mn == 0) continue;
             double *const D = (double *)((unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)dA, 8 * m) |
@@ -108,13 +109,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void po
 }
 
 template <int KM>
-void launch(hipStream_t st, const int *order, int count, const int *nsz, const double *const *L,
+void launch(hipStream_t st, int num_cus, const int *order, int count, const int *nsz, const double *const *L,
             const double *const *X, const double *const *dX, double *const *dA, double *const *dB, int nrhs)
 {
     const auto kernel = nrhs > 2 ? potrs_backward_kernel<KM, 4>
                       : nrhs > 1 ? potrs_backward_kernel<KM, 2> : potrs_backward_kernel<KM, 1>;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)nrocm_cdiv(count, 8)), dim3(64), 0, st, order, count, nsz, L, X, dX, dA,
-                       dB, nrhs);
+    const int per = members_per_wave(num_cus, count);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)nrocm_cdiv(count, per)), dim3(64), 0, st, order, count, per, nsz, L, X, dX,
+                       dA, dB, nrhs);
 }
 
 }  // namespace
@@ -135,9 +137,9 @@ extern "C" int nrocm_dpotrs_backward_batched(nrocm_handle h, nrocm_batch bt, con
         return nrocm_fail(h, NROCM_ERR_UNSUPPORTED, "batched Cholesky adjoint supports n <= 64");
     // `order` holds the members by decreasing size
     if (bt->max_n <= 32)
-        launch<4>(h->stream, bt->order_dev, bt->count, bt->n_dev, L, X, dX, dA, dB, bt->nrhs);
+        launch<4>(h->stream, h->num_cus, bt->order_dev, bt->count, bt->n_dev, L, X, dX, dA, dB, bt->nrhs);
     else
-        launch<8>(h->stream, bt->order_dev, bt->count, bt->n_dev, L, X, dX, dA, dB, bt->nrhs);
+        launch<8>(h->stream, h->num_cus, bt->order_dev, bt->count, bt->n_dev, L, X, dX, dA, dB, bt->nrhs);
     NROCM_CHECK_LAUNCH(h);
     return NROCM_OK;
 }

@@ -296,7 +296,7 @@ __global__ __launch_bounds__(64) void getrf_getrs_batched_kernel(
 //
 // Bound by the chain of dots, one per row: products, up to 8 additions, the
 // joining of the accumulators and the tail, about 300 cycles a step.  One
-// member's chain uses few lanes, so eight members share a wavefront (eight lanes
+// member's chain uses few lanes, so up to eight members share a wavefront (eight lanes
 // each, the accumulators of a dot side by side), nothing of a step crosses a
 // group, and no step needs a barrier; members of the whole range of sizes run in
 // one launch, the largest first.  Before, a member had 16 to 64 lanes, a dot
@@ -306,8 +306,8 @@ __global__ __launch_bounds__(64) void getrf_getrs_batched_kernel(
 // KM: blocks of 8 rows that a lane can hold; CH: right-hand sides at a time.
 template <int KM, int CH>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void getrs_backward_batched_kernel(
-    const int *__restrict__ order, int count, const int *__restrict__ nsz, const double *const *__restrict__ LUptr,
-    const int *const *__restrict__ Pptr, const double *const *__restrict__ Xptr,
+    const int *__restrict__ order, int count, int per, const int *__restrict__ nsz,
+    const double *const *__restrict__ LUptr, const int *const *__restrict__ Pptr, const double *const *__restrict__ Xptr,
     const double *const *__restrict__ dXptr, double *const *__restrict__ dAptr, double *const *__restrict__ dBptr,
     int nrhs)
 {
@@ -317,8 +317,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void ge
     __shared__ int swap[8][NB];
     const int lane = threadIdx.x;
     const int g = lane >> 3, c = lane & 7;
-    const int item = (int)blockIdx.x * 8 + g;
-    const bool valid = item < count;
+    const int item = (int)blockIdx.x * per + g;
+    const bool valid = g < per && item < count;
     const int jm = valid ? order[item] : 0;
     const int n = valid ? nsz[jm] : 0;
     int most = n;
@@ -376,7 +376,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void ge
             }
         __syncthreads();
         const unsigned long long dA = n > 0 ? (unsigned long long)dAptr[jm] : 0;
-        for (int m = 0; m < 8; ++m) {
+        for (int m = 0; m < per; ++m) {
             const int mn = __builtin_amdgcn_readlane(n, 8 * m);
             if (mn == 0) continue;
             double *const D = (double *)((unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)dA, 8 * m) |
@@ -407,17 +407,18 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void ge
 
 // One launch for the whole batch: `order` holds the members by decreasing size.
 template <int KM>
-void launch_bwd(hipStream_t st, const int *order, int count, const int *nsz, const double *const *LU,
+void launch_bwd(hipStream_t st, int num_cus, const int *order, int count, const int *nsz, const double *const *LU,
                 const int *const *P, const double *const *X, const double *const *dX, double *const *dA,
                 double *const *dB, int nrhs)
 {
-    const dim3 grid((unsigned)((count + 7) / 8));
+    const int per = members_per_wave(num_cus, count);
+    const dim3 grid(nrocm_cdiv(count, per));
     if (nrhs > 1)
-        hipLaunchKernelGGL((getrs_backward_batched_kernel<KM, 2>), grid, dim3(64), 0, st, order, count, nsz, LU, P, X,
-                           dX, dA, dB, nrhs);
+        hipLaunchKernelGGL((getrs_backward_batched_kernel<KM, 2>), grid, dim3(64), 0, st, order, count, per, nsz, LU, P,
+                           X, dX, dA, dB, nrhs);
     else
-        hipLaunchKernelGGL((getrs_backward_batched_kernel<KM, 1>), grid, dim3(64), 0, st, order, count, nsz, LU, P, X,
-                           dX, dA, dB, nrhs);
+        hipLaunchKernelGGL((getrs_backward_batched_kernel<KM, 1>), grid, dim3(64), 0, st, order, count, per, nsz, LU, P,
+                           X, dX, dA, dB, nrhs);
 }
 
 template <int NB>
@@ -487,9 +488,9 @@ extern "C" int nrocm_dgetrs_backward_batched(nrocm_handle h, nrocm_batch bt, con
     if (bt->max_n > 64) return nrocm_fail(h, NROCM_ERR_UNSUPPORTED, "batched LU adjoint supports n <= 64");
     // up to 32 rows a lane holds half as many values, and the dots have half the terms
     if (bt->max_n <= 32)
-        launch_bwd<4>(h->stream, bt->order_dev, bt->count, bt->n_dev, lu, ipiv, x, dx, da, db, bt->nrhs);
+        launch_bwd<4>(h->stream, h->num_cus, bt->order_dev, bt->count, bt->n_dev, lu, ipiv, x, dx, da, db, bt->nrhs);
     else
-        launch_bwd<8>(h->stream, bt->order_dev, bt->count, bt->n_dev, lu, ipiv, x, dx, da, db, bt->nrhs);
+        launch_bwd<8>(h->stream, h->num_cus, bt->order_dev, bt->count, bt->n_dev, lu, ipiv, x, dx, da, db, bt->nrhs);
     NROCM_CHECK_LAUNCH(h);
     return NROCM_OK;
 }
