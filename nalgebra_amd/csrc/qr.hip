@@ -611,6 +611,17 @@ int geqrf_columns(nrocm_handle h, int m, int n, T *a, int lda, T *diag)
     return NROCM_OK;
 }
 
+// Matrices whose columns take less time than the pipeline's hand-overs and the
+// filling of its buffer (f64, us, one workgroup and pipeline: 2 x 2 4.2 and 5.8, 4 x 4 8.4
+// and 9.6, 8 x 4 9.9 and 9.7, 5 x 5 10.8 and 15.3, 20 x 20 48.7 and 50.6, 24 x 24 61.0 and 60.4;
+// f32: 5 x 5 10.2 and 12.7, 12 x 12 24.8 and 25.6, 16 x 16 34.8 and 33.1).  Up to four columns
+// are one group and need no buffer.
+bool qr_is_tiny(int m, int n, bool f64)
+{
+    if (n <= 4) return n > 1 && m <= 4;
+    return std::max(m, n) <= (f64 ? 20 : 12);
+}
+
 // The column pipeline takes its hand-over buffer from the handle's workspace;
 // on a stream under capture, where that may not grow and must not be baked in,
 // and above the rows that registers hold, one workgroup walks the columns.
@@ -622,7 +633,7 @@ int geqrf(nrocm_handle h, int m, int n, T *a, int lda, T *diag)
         (void)hipGetLastError();  // the legacy stream beside a capture
         cap = hipStreamCaptureStatusActive;
     }
-    if (cap != hipStreamCaptureStatusNone || m > QR_COLUMNS_MAX) {
+    if (cap != hipStreamCaptureStatusNone || m > QR_COLUMNS_MAX || qr_is_tiny(m, n, sizeof(T) == 8)) {
         hipLaunchKernelGGL((geqrf_exact_kernel<T>), dim3(1), dim3(256), 0, h->stream, a, m, n, lda, diag);
         NROCM_CHECK_LAUNCH(h);
         return NROCM_OK;
