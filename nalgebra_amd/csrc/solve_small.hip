@@ -4,7 +4,7 @@
 // A workgroup takes CH right-hand sides through the whole solve, its four
 // wavefronts the 64-row blocks in turn (solve_sweep.hpp); everything it
 // exchanges is in its own LDS, so calls on several streams share nothing.
-// 300 right-hand sides are 75 workgroups instead of 300 solves in a row:
+// 300 right-hand sides are 150 workgroups of two instead of 300 solves in a row:
 // n = 300 with 300 right-hand sides 124.8 ms -> 60 us, n = 500 with one
 // 827 -> 72 us (before: one workgroup, a barrier and a load per step).
 #include "internal_launch.hpp"
@@ -139,6 +139,79 @@ __global__ __launch_bounds__(THREADS) void solve_small_kernel(const double *__re
     }
 }
 
+// Up to TINY rows a thread takes a right-hand side through the whole solve, matrix
+// and vector in registers: the launch and one trip to memory are all there is.  (LU,
+// EXACT, one right-hand side, us, with the kernel above and this one: n = 1 6.2 and 4.1,
+// 4 6.4 and 4.3, 8 7.0 and 5.0; Cholesky 4 6.5 and 4.0, 8 8.3 and 4.0.)
+constexpr int TINY = 8;
+
+template <bool EXACT, int OP>
+__global__ __launch_bounds__(64) void solve_tiny_kernel(const double *__restrict__ M, int lda, int n,
+                                                        const int *__restrict__ ipiv, const double *__restrict__ dg,
+                                                        double *B, int ldb, int nrhs, int *info)
+{
+    const int c = blockIdx.x * 64 + threadIdx.x;
+    double *const b = B + (size_t)min(c, nrhs - 1) * ldb;
+    double m[TINY][TINY], x[TINY], d[TINY];  // m[j][i]: element (i, j)
+    int p[TINY];
+#pragma unroll
+    for (int j = 0; j < TINY; ++j) {
+#pragma unroll
+        for (int i = 0; i < TINY; ++i) m[j][i] = M[min(i, n - 1) + (size_t)min(j, n - 1) * lda];
+        x[j] = b[min(j, n - 1)];
+        d[j] = OP == OP_QR ? fabs(dg[min(j, n - 1)]) : m[j][j];
+        p[j] = OP == OP_LU ? ipiv[min(j, n - 1)] : j;
+    }
+    if constexpr (OP == OP_LU) {
+#pragma unroll
+        for (int i = 0; i < TINY; ++i) {
+            if (i >= n) break;
+            double t = x[i];
+#pragma unroll
+            for (int j = 0; j < TINY; ++j) t = j == p[i] && j < n ? x[j] : t;
+#pragma unroll
+            for (int j = 0; j < TINY; ++j) x[j] = j == p[i] && j < n ? x[i] : x[j];
+            x[i] = t;
+        }
+    }
+    auto axpy = [&](int r, int i, double a) {
+        double acc[1] = {x[r]};
+        const double f[1] = {x[i]};
+        step<EXACT, 1>(acc, f, a);
+        x[r] = acc[0];
+    };
+    if constexpr (OP != OP_QR) {
+#pragma unroll
+        for (int i = 0; i < TINY; ++i) {
+            if (i >= n) break;
+            if constexpr (OP == OP_CHOL) x[i] = x[i] / d[i];
+#pragma unroll
+            for (int r = i + 1; r < TINY; ++r) axpy(r, i, m[i][r]);
+        }
+    }
+    int fail = 0;
+#pragma unroll
+    for (int i = TINY - 1; i >= 0; --i) {
+        if (i >= n) continue;
+        if constexpr (OP == OP_CHOL && EXACT) {
+            double res = 0.0;  // dotx of fewer than eight elements
+#pragma unroll
+            for (int e = i + 1; e < TINY; ++e)
+                if (e < n) res += m[i][e] * x[e];
+            x[i] = (x[i] - res) / d[i];
+        } else {
+            if (d[i] == 0.0 && fail == 0) fail = i + 1;
+            x[i] = x[i] / d[i];
+#pragma unroll
+            for (int r = 0; r < i; ++r) axpy(r, i, OP == OP_CHOL ? m[r][i] : m[i][r]);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < TINY; ++i)
+        if (i < n && c < nrhs) b[i] = x[i];
+    if (OP != OP_CHOL && info && c == 0) *info = fail;
+}
+
 __global__ void zero_info_kernel(int *info) { *info = 0; }
 
 template <bool EXACT, int OP, int CH>
@@ -164,11 +237,18 @@ int solve_small(nrocm_handle h, const double *M, int lda, int n, const int *ipiv
         }
         return NROCM_OK;
     }
+    if (n <= TINY) {
+        const auto kernel = exact ? solve_tiny_kernel<true, OP> : solve_tiny_kernel<OP == OP_QR, OP>;  // QR: always exact
+        hipLaunchKernelGGL(kernel, dim3(nrocm_cdiv(nrhs, 64)), dim3(64), 0, h->stream, M, lda, n, ipiv, dg, B, ldb,
+                           nrhs, info);
+        NROCM_CHECK_LAUNCH(h);
+        return NROCM_OK;
+    }
     // fewer right-hand sides per workgroup where the LDS does not hold them
     // (QR's solve above n = 2,900)
 #define NROCM_SMALL(CH)                                                                       \
     (exact ? launch<true, OP, CH>(h, M, lda, n, ipiv, dg, B, ldb, nrhs, info)                 \
-           : launch<false, OP, CH>(h, M, lda, n, ipiv, dg, B, ldb, nrhs, info))
+           : launch<OP == OP_QR, OP, CH>(h, M, lda, n, ipiv, dg, B, ldb, nrhs, info))
     const int fit = lds_bytes(n, 4, OP, exact) <= LDS_MOST ? 4 : lds_bytes(n, 2, OP, exact) <= LDS_MOST ? 2 : 1;
     const int ch = std::min(fit, rhs_per_group(h->num_cus, nrhs, 1));
     return ch == 1 ? NROCM_SMALL(1) : ch == 2 ? NROCM_SMALL(2) : NROCM_SMALL(4);
