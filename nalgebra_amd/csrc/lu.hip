@@ -51,11 +51,11 @@ struct LuBuffer {
     size_t bytes() const { return LU_HEADER_BYTES + parts * part_words() * sizeof(U); }
     U *V(int c0) const { return words + (size_t)(c0 / LU_NB % parts) * part_words(); }
     U *H(int c0) const { return V(c0) + (size_t)cols * ldv; }
-    hipError_t clear(hipStream_t st)  // the first part
+    hipError_t clear(hipStream_t st, int *info)  // the first part, and info
     {
         const size_t count = part_words();
         hipLaunchKernelGGL((fill_words_kernel<U>), dim3(std::min<size_t>(4096, nrocm_cdiv(count, 1024) + 4)), dim3(256),
-                           0, st, words, count, ColWord<T>::EMPTY, tickets, (int)(LU_HEADER_BYTES / sizeof(int)));
+                           0, st, words, count, ColWord<T>::EMPTY, tickets, (int)(LU_HEADER_BYTES / sizeof(int)), info);
         return hipGetLastError();
     }
 };
@@ -169,7 +169,7 @@ int getrf_whole(nrocm_handle h, hipStream_t st, int m, int n, T *A, int lda, int
 {
     LuBuffer<T> b(buf, m, n);
     const int mn = std::min(m, n);
-    LU_TRY(b.clear(st));
+    LU_TRY(b.clear(st, info));
     LU_TRY(lu_columns<T>(st, A, lda, m, 0, n, mn, ipiv, info, b, 0, nrocm_wait_limit(h, COL_SPIN_LIMIT)));
     LU_TRY(lu_left<T>(st, A, lda, m, 0, mn, ipiv, b, false));
     return NROCM_OK;
@@ -184,7 +184,7 @@ int getrf_panels(nrocm_handle h, hipStream_t st, int m, int n, T *A, int lda, in
     const bool exact = trail == TRAIL_EXACT;
     constexpr int NB = LU_NB;
     const long limit = nrocm_wait_limit(h, COL_SPIN_LIMIT);
-    LU_TRY(b.clear(st));
+    LU_TRY(b.clear(st, info));
     LU_TRY(lu_columns<T>(st, A, lda, m, 0, std::min(NB, mn), std::min(NB, mn), ipiv, info, b, 0, limit));
     for (int j0 = 0; j0 < mn; j0 += NB) {
         const int nb = std::min(NB, mn - j0), j1 = j0 + nb;
@@ -500,8 +500,6 @@ int getrf_graph(nrocm_handle h, int m, int n, T *A, int lda, int *ipiv, int *inf
     void *buf = nullptr;
     int s = nrocm_workspace(h, LuBuffer<T>(nullptr, m, n).bytes(), &buf, NROCM_WS_LU);
     if (s != NROCM_OK) return s;
-    hipLaunchKernelGGL(fill_int_kernel, dim3(1), dim3(64), 0, h->stream, info, 1, 0);
-    NROCM_CHECK_LAUNCH(h);
     if (lu_is_whole(m, n)) return getrf_whole<T>(h, h->stream, m, n, A, lda, ipiv, info, buf);
     s = nrocm_aux_init(h);  // streams and events exist before the capture
     if (s != NROCM_OK) return s;

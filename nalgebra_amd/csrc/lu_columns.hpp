@@ -467,9 +467,10 @@ __global__ __launch_bounds__(512) void swap_rows_kernel(T *A, int lda, int m, co
 }
 
 template <typename U>
-__global__ void fill_words_kernel(U *p, size_t count, U v, int *ints, int nints)
+__global__ void fill_words_kernel(U *p, size_t count, U v, int *ints, int nints, int *info)
 {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i == 0) *info = 0;
     if (i < (size_t)nints) ints[i] = 0;
     for (size_t e = i; e < count; e += (size_t)gridDim.x * blockDim.x) p[e] = v;
 }
