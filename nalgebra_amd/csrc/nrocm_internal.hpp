@@ -109,7 +109,8 @@ struct nrocm_handle_s {
 static inline long nrocm_wait_limit(nrocm_handle h, long usual) { return h->wait_polls > 0 ? h->wait_polls : usual; }
 
 // Runs `body(stream)` through the handle's graph cache: on a miss the launches
-// are captured into a new graph; either way the graph is launched on h->stream.
+// are captured into a new graph; either way the graph is launched on h->stream
+// (under capture the body runs on h->stream itself).
 template <typename F>
 int nrocm_graph_run(nrocm_handle h, const long long (&key)[8], F body);
 
@@ -182,6 +183,14 @@ static inline unsigned nrocm_cdiv(size_t a, size_t b) { return (unsigned)((a + b
 template <typename F>
 int nrocm_graph_run(nrocm_handle h, const long long (&key)[8], F body)
 {
+    // A graph launched on a stream under capture does not become part of the
+    // caller's graph: there the launches themselves are captured.
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(h->stream, &cap) != hipSuccess) {
+        (void)hipGetLastError();  // the legacy stream beside a capture
+        cap = hipStreamCaptureStatusNone;
+    }
+    if (cap != hipStreamCaptureStatusNone) return body(h->stream);
     nrocm_handle_s::Graph *hit = nullptr;
     for (auto &g : h->graphs) {
         bool same = true;

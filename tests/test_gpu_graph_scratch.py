@@ -105,3 +105,24 @@ def test_graph_scratch_is_given_back(nl):
     assert free0 - torch.cuda.mem_get_info()[0] < calls * n * n * 4
     assert L.nrocm_free_graph_scratch(None) == -1
     assert L.nrocm_destroy(h) == 0
+
+
+@pytest.mark.parametrize("n,mode", [(1100, 0), (2300, 1)])
+def test_captured_lu_of_panels(nl, n, mode):
+    """Above 1024 rows the factorisation is many launches on two streams."""
+    a = nl.DMatrix(torch.rand(n * n, dtype=torch.float64, device="cuda").sub_(0.5), n, n)
+    ref = a.lu(mode)
+    buf = nl.DMatrix(torch.empty_like(a.data), n, n)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        buf.data.copy_(a.data)
+        lu = nl.LU(buf, mode)
+    for _ in range(3):
+        buf.data.zero_()
+        lu.ipiv.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(lu.lu.data, ref.lu.data) and torch.equal(lu.ipiv, ref.ipiv) and lu.info == 0
+        other = a.lu(mode)  # eager, between the replays
+        torch.cuda.synchronize()
+        assert torch.equal(other.lu.data, ref.lu.data)
