@@ -421,7 +421,8 @@ int nrocm_dpotrf_potrs_batched(nrocm_handle h, nrocm_batch bt, double *const *A,
     if (bt->max_n > 64)
         return nrocm_fail(h, NROCM_ERR_UNSUPPORTED, "batched Cholesky supports n <= 64");
     const bool exact = mode == NROCM_EXACT;
-    if (!bt->use_graph) return launch_batched(h, bt, h->stream, A, B, info, exact);
+    // under capture the launches themselves become part of the caller's graph
+    if (!bt->use_graph || nrocm_capturing(h)) return launch_batched(h, bt, h->stream, A, B, info, exact);
 
     const void *key[3] = {A, B, info};
     nrocm_batch_s::GraphEntry *hit = nullptr;

@@ -180,17 +180,23 @@ int nrocm_join_on(nrocm_handle h, hipStream_t st, int count);
 
 static inline unsigned nrocm_cdiv(size_t a, size_t b) { return (unsigned)((a + b - 1) / b); }
 
+// Is the handle's stream recording a caller's graph?
+static inline bool nrocm_capturing(nrocm_handle h)
+{
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(h->stream, &cap) != hipSuccess) {
+        (void)hipGetLastError();  // the legacy stream beside a capture
+        return false;
+    }
+    return cap != hipStreamCaptureStatusNone;
+}
+
 template <typename F>
 int nrocm_graph_run(nrocm_handle h, const long long (&key)[8], F body)
 {
     // A graph launched on a stream under capture does not become part of the
     // caller's graph: there the launches themselves are captured.
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(h->stream, &cap) != hipSuccess) {
-        (void)hipGetLastError();  // the legacy stream beside a capture
-        cap = hipStreamCaptureStatusNone;
-    }
-    if (cap != hipStreamCaptureStatusNone) return body(h->stream);
+    if (nrocm_capturing(h)) return body(h->stream);
     nrocm_handle_s::Graph *hit = nullptr;
     for (auto &g : h->graphs) {
         bool same = true;

@@ -126,3 +126,32 @@ def test_captured_lu_of_panels(nl, n, mode):
         other = a.lu(mode)  # eager, between the replays
         torch.cuda.synchronize()
         assert torch.equal(other.lu.data, ref.lu.data)
+
+
+def test_captured_batches(nl):
+    """The batched Cholesky replays a graph of its own when it is not captured."""
+    import gen
+    ns = [4, 17, 33, 64, 9, 30, 50] * 20
+    A, _, B, _ = gen.spd_batch(5, ns, 2)
+    bt = nl.CholeskyBatch(ns, 2)
+    A0, B0 = torch.from_numpy(A).cuda(), torch.from_numpy(B).cuda()
+    a, b = A0.clone(), B0.clone()
+    ptrs = bt.pointers(a, b)
+    info = torch.ones(len(ns), dtype=torch.int32, device="cuda")
+    bt.solve_ptrs(*ptrs, info)  # eager
+    torch.cuda.synchronize()
+    want = [a.clone(), b.clone()]
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        a.copy_(A0)
+        b.copy_(B0)
+        bt.solve_ptrs(*ptrs, info)
+    for _ in range(3):
+        a.zero_(), b.zero_(), info.fill_(1)
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(a, want[0]) and torch.equal(b, want[1]) and not info.any()
+        a.copy_(A0), b.copy_(B0)
+        bt.solve_ptrs(*ptrs, info)
+        torch.cuda.synchronize()
+        assert torch.equal(b, want[1])
