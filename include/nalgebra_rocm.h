@@ -105,6 +105,8 @@ int nrocm_sgemm(nrocm_handle handle, size_t m, size_t k, size_t n, float alpha,
  * src/linalg/permutation_sequence.rs:84-93).  info[0] = 0, or 1 + the first
  * step whose column was entirely zero (nalgebra skips it, lu.rs:107-110), or
  * -1 if an internal wait timed out (nrocm_set_wait_limit).
+ * Scratch: up to 1024 rows, or with min(m, n) <= 64, as much as the matrix's first
+ * min(m, n) columns; else two panels of 64 columns.
  * Shape of nalgebra-lapack's LUScalar::xgetrf (nalgebra-lapack/src/lu.rs:351-380). */
 int nrocm_dgetrf(nrocm_handle handle, int m, int n, double *a, int lda, int *ipiv,
                  int *info, int mode);
@@ -112,7 +114,8 @@ int nrocm_dgetrf(nrocm_handle handle, int m, int n, double *a, int lda, int *ipi
 /* LU::solve_mut (lu.rs:242-260): B (n x nrhs) <- A^{-1} B.  info[0] = 0, or
  * 1 + the index of an exact zero on U's diagonal (solve_mut returns false and
  * B holds garbage); the n >= 1024 path also reports -1 if an internal wait
- * timed out and -2 for a pivot outside [0, n) (not applied).  Any n (n >= 1024: one 64-row block per workgroup, pipelined).
+ * timed out and -2 for a pivot outside [0, n) (not applied).  Any n (n >= 1024: four 64-row blocks
+ * per workgroup, pipelined).
  * Shape of LUScalar::xgetrs. */
 int nrocm_dgetrs(nrocm_handle handle, int n, int nrhs, const double *lu, int lda,
                  const int *ipiv, double *b, int ldb, int *info, int mode);
@@ -151,9 +154,10 @@ int nrocm_dpotrf_substitute(nrocm_handle handle, int n, double *a, int lda, doub
  * cholesky.rs:166-184; ln is the device's, within 1 ulp of libm's). */
 int nrocm_ddiag_det(nrocm_handle handle, int n, const double *a, int lda, double *out);
 /* Cholesky::solve_mut (cholesky.rs:122-129): B <- (L L^T)^{-1} B, any n.
- * n >= 1024: the forward sweep runs one 64-row block per workgroup; the
+ * n >= 1024: the forward sweep runs four 64-row blocks per workgroup; the
  * EXACT transposed solve keeps nalgebra's dot order, one dependent chain of
- * about n^2/16 additions on one wavefront. */
+ * about n^2/16 additions on one wavefront, which seven others feed up to
+ * n = 4096 (above that it reads L by itself, one right-hand side after another). */
 int nrocm_dpotrs(nrocm_handle handle, int n, int nrhs, const double *l, int lda,
                  double *b, int ldb, int mode);
 
@@ -244,7 +248,9 @@ int nrocm_dpotrs_backward_batched(nrocm_handle handle, nrocm_batch batch,
 /* ---------------------------------------------------------------- QR (a10-a12)
  * QR::new (src/linalg/qr.rs:55-76): column i of A holds the unit Householder
  * axis in rows i..m, diag[i] the signed norm (R_ii = |diag[i]|, qr.rs:81-89),
- * the strict upper triangle holds R.  Exact nalgebra arithmetic. */
+ * the strict upper triangle holds R.  Exact nalgebra arithmetic.  Scratch: as much
+ * as the matrix's first min(m, n) columns (none up to 20 x 20, f32 12 x 12, above
+ * 16384 rows and under capture, where one workgroup takes the columns in turn). */
 int nrocm_dgeqrf(nrocm_handle handle, int m, int n, double *a, int lda, double *diag);
 int nrocm_sgeqrf(nrocm_handle handle, int m, int n, float *a, int lda, float *diag);
 /* QR::q_tr_mul (qr.rs:157-171): B (m x nrhs) <- Q^T B. */

@@ -672,7 +672,9 @@ hipError_t gemm_cm_launch(hipStream_t st, int m, int n, int k, TS alpha, const T
 // the split-k shape, or, where C has at most two 16 x 16 tiles per CU, no
 // staging at all (f64, us, staged and direct: 300^3, 361 tiles, 18.3 and 8.5;
 // 400^3, 625 tiles, 19.1 and 18.5; 512^3, 1024 tiles, 19.7 and 24.1; f32 at 625
-// tiles already 14.5 and 16.3).
+// tiles already 14.5 and 16.3; long k near the line, 484 tiles: 352 x 20000 x 352
+// f64 561 and 343, f32 303 and 291, 352 x 512 x 352 f32 11.1 and 11.3; 512 tiles in a row,
+// 16 x 4096 x 8192 f32 175 and 63).
 template <typename TS, int MODE>
 hipError_t gemm_cm(hipStream_t st, int m, int n, int k, TS alpha, const TS *A, long lda, const TS *B, long ldb,
                    TS beta, TS *C, long ldc)

@@ -24,7 +24,9 @@ namespace {
 // Whole matrices of up to this many rows are one pipeline; above it every group
 // takes too long to catch up with all the earlier ones (EXACT, one pipeline
 // against 64-column panels: n = 700 1.19 and 1.42 ms, 1000 1.94 and 2.15, 1100
-// 2.97 and 2.51, 2048 8.2 and 5.3).
+// 2.97 and 2.51, 2048 8.2 and 5.3).  FAST and wide matrices take the same rule,
+// measured against the panels that came before these pipelines: 1000 x 1000 FAST 1.91
+// and 4.45 ms, 1000 x 4096 3.67 and 4.73, 1000 x 16384 5.78 and 5.74.
 constexpr int WHOLE_ROWS = 1024;
 
 // The pipeline's buffer, after a header of one ticket per panel: L columns and
@@ -434,7 +436,7 @@ hipError_t window_panel(hipStream_t st, T *A, int lda, int n, int k0, int *ipiv,
 // Blocked LU with the pivot search of each 64-column block restricted to a
 // window of WINDOW_ROWS rows (window_panel_kernel), then the window's row
 // plan on the other columns, A21 U11^{-1} for the rows below the window, U12
-// and the trailing update.  ipiv has the LAPACK meaning, as for getrf_impl;
+// and the trailing update.  ipiv has the LAPACK meaning, as for getrf_panels;
 // perm (optional) receives the composed row permutation.
 //
 // Look-ahead of depth one: the panel step of block k+1 needs only the

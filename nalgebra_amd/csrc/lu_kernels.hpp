@@ -346,7 +346,7 @@ __device__ __forceinline__ unsigned pivot_key(T av, int pos)
 }
 
 // Wavefront maximum of an unsigned value; lane 63 ends with it (same DPP
-// pattern as argmax_wave).
+// pattern as max_wave).
 __device__ __forceinline__ unsigned wave_max_u32(unsigned k)
 {
     k = max(k, (unsigned)dpp32<0x111, 0xf>(0, (int)k));

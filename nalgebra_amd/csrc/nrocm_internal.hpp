@@ -28,13 +28,15 @@ __device__ __forceinline__ void lds_barrier()
 #ifdef __HIPCC__
 constexpr size_t NROCM_LDS_BYTES = 160 * 1024;  // of one CU (gfx950), static and dynamic together
 
+constexpr int NROCM_DEVICES = 64;  // that a process may use
+
 // Lets kernel K be launched with dynamic LDS beyond the runtime's default (all
-// that its static LDS leaves).
+// that its static LDS leaves) on the current device.
 template <auto K>
-void nrocm_allow_lds()
+void nrocm_allow_lds(int device)
 {
-    static std::once_flag once;
-    std::call_once(once, [] {
+    static std::once_flag once[NROCM_DEVICES];
+    std::call_once(once[device % NROCM_DEVICES], [] {
         hipFuncAttributes a;
         if (hipFuncGetAttributes(&a, (const void *)K) == hipSuccess && a.sharedSizeBytes < NROCM_LDS_BYTES)
             (void)hipFuncSetAttribute((const void *)K, hipFuncAttributeMaxDynamicSharedMemorySize,

@@ -603,7 +603,7 @@ int geqrf_columns(nrocm_handle h, int m, int n, T *a, int lda, T *diag)
         hipLaunchKernelGGL((qr_prep_kernel<U>), dim3(std::min(2048u, nrocm_cdiv(words, 512))), dim3(256), 0, h->stream,
                            V, words, Word<T>::EMPTY, ticket);
     }
-    nrocm_allow_lds<geqrf_columns_kernel<T, RPT, PC>>();
+    nrocm_allow_lds<geqrf_columns_kernel<T, RPT, PC>>(h->device);
     hipLaunchKernelGGL((geqrf_columns_kernel<T, RPT, PC>), dim3(groups), dim3(PT),
                        qr_lds_elements(m, PC) * sizeof(T), h->stream, a, m, n, lda, diag, V, H, ticket,
                        nrocm_wait_limit(h, QR_SPIN_LIMIT));
@@ -650,7 +650,7 @@ template <int RPT, int PC, bool REVERSE>
 int qr_apply_columns(nrocm_handle h, int m, int n, const double *qr, int lda, const double *diag, int nrhs, double *b,
                      int ldb)
 {
-    nrocm_allow_lds<qr_apply_kernel<RPT, PC, REVERSE>>();
+    nrocm_allow_lds<qr_apply_kernel<RPT, PC, REVERSE>>(h->device);
     hipLaunchKernelGGL((qr_apply_kernel<RPT, PC, REVERSE>), dim3(nrocm_cdiv(nrhs, PC)), dim3(PT),
                        qr_lds_elements(m, PC) * sizeof(double), h->stream, qr, m, n, lda, diag, b, ldb, nrhs);
     NROCM_CHECK_LAUNCH(h);

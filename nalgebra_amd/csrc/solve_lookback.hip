@@ -313,7 +313,7 @@ int chol_dot(nrocm_handle h, hipStream_t st, const double *L, int lda, int n, do
         const dim3 grid(nrocm_cdiv(nrhs, ch));
 #define NROCM_DOT(NR, CH)                                                                                 \
     do {                                                                                                  \
-        nrocm_allow_lds<chol_dot_kernel<NR, CH>>();                                                       \
+        nrocm_allow_lds<chol_dot_kernel<NR, CH>>(h->device);                                                       \
         hipLaunchKernelGGL((chol_dot_kernel<NR, CH>), grid, dim3(512), lds, st, L, lda, n, b, ldb, nrhs);  \
     } while (0)
         if (n <= 2048) {
@@ -329,7 +329,7 @@ int chol_dot(nrocm_handle h, hipStream_t st, const double *L, int lda, int n, do
         return NROCM_OK;
     }
     const bool lds = n <= CHOL_XS_LDS_MAX;
-    if (lds) nrocm_allow_lds<chol_backward_dot_kernel<true>>();
+    if (lds) nrocm_allow_lds<chol_backward_dot_kernel<true>>(h->device);
     for (int c = 0; c < nrhs; ++c) {
         double *bc = b + (size_t)c * ldb;
         if (lds)
@@ -361,7 +361,7 @@ int solve(nrocm_handle h, hipStream_t st, int n, int nrhs, const double *M, int 
         // and info are made once
         const int *piv = c0 == 0 ? ipiv : nullptr;
         const unsigned blocks = std::min<unsigned>(512, std::max(1u, nrocm_cdiv(ntag, PREP_WAVES * 64 * 4)));
-        nrocm_allow_lds<prep_kernel>();
+        nrocm_allow_lds<prep_kernel>(h->device);
         hipLaunchKernelGGL(prep_kernel, dim3(blocks), dim3(PREP_WAVES * 64),
                            piv && n <= PERM_LDS_MAX ? (size_t)n * sizeof(int) : 0, st, tags, ntag, header, info,
                            c0 == 0 && info, piv, n, perm);

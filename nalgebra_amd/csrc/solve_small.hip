@@ -219,7 +219,7 @@ int launch(nrocm_handle h, const double *M, int lda, int n, const int *ipiv, con
            int nrhs, int *info)
 {
     const size_t lds = lds_bytes(n, CH, OP, EXACT);
-    nrocm_allow_lds<solve_small_kernel<EXACT, OP, CH>>();
+    nrocm_allow_lds<solve_small_kernel<EXACT, OP, CH>>(h->device);
     hipLaunchKernelGGL((solve_small_kernel<EXACT, OP, CH>), dim3(nrocm_cdiv(nrhs, CH)), dim3(THREADS), lds, h->stream,
                        M, lda, n, ipiv, dg, B, ldb, nrhs, info);
     NROCM_CHECK_LAUNCH(h);
